@@ -65,6 +65,33 @@ struct Part {
 SGEMM_INTERNAL int decompose(const sgemm_handle* h, uint32_t m, uint32_t n, uint32_t k, uint32_t lda, uint32_t ldb,
                              uint32_t ldc, uint32_t ldd, Part out[3]);
 
+// How a launch runs on the split-BF16 kernels (bf16x6_plan.hpp): `tile` of
+// kTiles over m x n (the whole problem, or its whole tiles where the handle's
+// edge kernels take thin strips) in `splits` K ranges; tile < 0: not at all.
+struct SplitPlan {
+    int tile = -1;
+    uint32_t splits = 1;
+    uint32_t m = 0, n = 0;
+    size_t partial_bytes = 0;
+    size_t ticket_count = 0;
+};
+SGEMM_INTERNAL SplitPlan split_plan(const sgemm_handle* h, uint32_t m, uint32_t n, uint32_t k, uint32_t lda, uint32_t ldb,
+                                    uint32_t ldc, uint32_t ldd, float alpha, float beta);
+// The strips of a split plan beside its m x n, on h's edge kernels.  Returns 0..2.
+SGEMM_INTERNAL int split_strips(const sgemm_handle* h, const SplitPlan& p, uint32_t m, uint32_t n, uint32_t lda,
+                                uint32_t ldb, uint32_t ldc, uint32_t ldd, Part out[2]);
+// Enqueues one checked split-BF16 launch; partials and tickets (zero, left
+// zero) only for splits > 1.  Weak: a program that holds only the host part
+// of the library has none, and its handles run their FP32 kernels.
+SGEMM_INTERNAL __attribute__((weak)) int bf16x6_launch(int tile, uint32_t splits, bool trans_a, bool trans_b,
+                                                       const float* dA, const float* dB, const float* dC, float* dD,
+                                                       uint32_t m, uint32_t n, uint32_t k, uint32_t lda, uint32_t ldb,
+                                                       uint32_t ldc, uint32_t ldd, float alpha, float beta,
+                                                       float* partials, uint32_t* tickets, hipStream_t stream);
+// Loads the split-BF16 kernels on the current device, so that no launch
+// (maybe under graph capture) does.
+SGEMM_INTERNAL __attribute__((weak)) int bf16x6_prepare();
+
 // Looks up the device address of sgemm_launch_noalloc's static scratch on
 // device `dev` (once per device; later calls return at once).  sgemm_open
 // calls it for the handle's device, so launches never do.
@@ -72,6 +99,8 @@ SGEMM_INTERNAL int noalloc_prepare(int dev);
 
 SGEMM_INTERNAL hipStream_t stream(const sgemm_handle* h);
 SGEMM_INTERNAL int device(const sgemm_handle* h);
+SGEMM_INTERNAL bool trans_a(const sgemm_handle* h);
+SGEMM_INTERNAL bool trans_b(const sgemm_handle* h);
 // Records `message` as the calling thread's sgemm_last_error and returns `code`.
 SGEMM_INTERNAL int set_error(int code, const char* message);
 

@@ -14,12 +14,16 @@
 // launch -- even the first one on a device, even under graph capture -- only
 // reads the stored pointer.
 
+#include "bf16x6_plan.hpp"
 #include "sgemm_internal.hpp"
 
 #include <hip/hip_runtime.h>
 
 #include <cstdio>
 #include <mutex>
+
+static_assert(bf16x6::kMaxPartialBytes <= SGEMM_NOALLOC_PARTIAL_BYTES && bf16x6::kMaxTickets <= SGEMM_NOALLOC_MAX_TILES,
+              "every split-BF16 plan fits the static scratch");
 
 namespace {
 
@@ -66,6 +70,21 @@ int scratch_address(int dev, void** out) {
     return SGEMM_OK;
 }
 
+// The scratch of h's device, its first `count` tickets cleared on `s`.
+int take_scratch(const sgemm_handle* h, size_t count, hipStream_t s, float** partials, uint32_t** tickets) {
+    void* base = nullptr;
+    const int r = scratch_address(sgemm_internal::device(h), &base);
+    if (r != SGEMM_OK) return r;
+    *partials = static_cast<float*>(base);
+    *tickets = reinterpret_cast<uint32_t*>(static_cast<unsigned char*>(base) + SGEMM_NOALLOC_PARTIAL_BYTES);
+    hipLaunchKernelGGL(clear_tickets, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, s, *tickets, (uint32_t)count);
+    const hipError_t e = hipGetLastError();
+    if (e == hipSuccess) return SGEMM_OK;
+    char msg[256];
+    snprintf(msg, sizeof(msg), "clear_tickets launch failed: %s (%d)", hipGetErrorString(e), (int)e);
+    return sgemm_internal::set_error((int)e, msg);
+}
+
 }  // namespace
 
 int sgemm_internal::noalloc_prepare(int dev) {
@@ -81,7 +100,10 @@ extern "C" int sgemm_launch_noalloc(sgemm_handle* h, const float* dA, const floa
     if (r != SGEMM_OK || m == 0 || n == 0) return r;
     hipStream_t s = sgemm_internal::stream(h);
     sgemm_internal::Part parts[3];
-    const int count = sgemm_internal::decompose(h, m, n, k, lda, ldb, ldc, ldd, parts);
+    // the split-BF16 plan never needs more than the scratch
+    const sgemm_internal::SplitPlan sp = sgemm_internal::split_plan(h, m, n, k, lda, ldb, ldc, ldd, alpha, beta);
+    const int count = sp.tile >= 0 ? sgemm_internal::split_strips(h, sp, m, n, lda, ldb, ldc, ldd, parts)
+                                   : sgemm_internal::decompose(h, m, n, k, lda, ldb, ldc, ldd, parts);
     // every part's needs are checked before anything is launched
     for (int q = 0; q < count; ++q) {
         const sgemm_internal::Part& pt = parts[q];
@@ -97,6 +119,14 @@ extern "C" int sgemm_launch_noalloc(sgemm_handle* h, const float* dA, const floa
             return sgemm_internal::set_error(SGEMM_E_SHAPE, msg);
         }
     }
+    if (sp.tile >= 0) {
+        float* partials = nullptr;
+        uint32_t* tickets = nullptr;
+        if (sp.partial_bytes && (r = take_scratch(h, sp.ticket_count, s, &partials, &tickets)) != SGEMM_OK) return r;
+        r = sgemm_internal::bf16x6_launch(sp.tile, sp.splits, sgemm_internal::trans_a(h), sgemm_internal::trans_b(h), dA,
+                                          dB, dC, dD, sp.m, sp.n, k, lda, ldb, ldc, ldd, alpha, beta, partials, tickets, s);
+        if (r != SGEMM_OK) return r;
+    }
     for (int q = 0; q < count; ++q) {
         const sgemm_internal::Part& pt = parts[q];
         const float* a = dA ? dA + pt.a_off : dA;
@@ -109,20 +139,10 @@ extern "C" int sgemm_launch_noalloc(sgemm_handle* h, const float* dA, const floa
             if (r != SGEMM_OK) return r;
             continue;
         }
-        void* base = nullptr;
-        if ((r = scratch_address(sgemm_internal::device(h), &base)) != SGEMM_OK) return r;
-        float* partials = static_cast<float*>(base);
-        uint32_t* tickets =
-            reinterpret_cast<uint32_t*>(static_cast<unsigned char*>(base) + SGEMM_NOALLOC_PARTIAL_BYTES);
+        float* partials = nullptr;
+        uint32_t* tickets = nullptr;
         // the parts run in order on one stream, so they share the scratch
-        hipLaunchKernelGGL(clear_tickets, dim3((unsigned)((p.ticket_count + 255) / 256)), dim3(256), 0, s, tickets,
-                           (uint32_t)p.ticket_count);
-        const hipError_t e = hipGetLastError();
-        if (e != hipSuccess) {
-            char msg[256];
-            snprintf(msg, sizeof(msg), "clear_tickets launch failed: %s (%d)", hipGetErrorString(e), (int)e);
-            return sgemm_internal::set_error((int)e, msg);
-        }
+        if ((r = take_scratch(h, p.ticket_count, s, &partials, &tickets)) != SGEMM_OK) return r;
         const sgemm_internal::Workspace ws{partials, (size_t)SGEMM_NOALLOC_PARTIAL_BYTES, tickets,
                                            (size_t)SGEMM_NOALLOC_MAX_TILES};
         r = sgemm_internal::launch(pt.kh, a, b, c, d, pt.m, pt.n, k, lda, ldb, ldc, ldd, alpha, beta, &ws, s);

@@ -6,6 +6,7 @@
 
 #include "sgemm_shim.h"
 #include "sgemm_internal.hpp"
+#include "bf16x6_plan.hpp"
 
 #include <hip/hip_runtime_api.h>
 
@@ -181,7 +182,7 @@ int toml_arr(const std::map<std::string, TomlValue>& t, const char* key, int* ou
         if (r_ != SGEMM_OK) return r_; \
     } while (0)
 
-int load_config(const char* path, sgemm_kernel_info* info) {
+int load_config(const char* path, sgemm_kernel_info* info, bool* split_bf16) {
     std::map<std::string, TomlValue> t;
     CFG_TRY(parse_toml(path, &t));
     int a_type, b_type, cd_type, scalar_type;
@@ -210,6 +211,11 @@ int load_config(const char* path, sgemm_kernel_info* info) {
     if (info->stream_k_rounds < 0) return fail(SGEMM_E_CONFIG, "stream_k_rounds = %d < 0", info->stream_k_rounds);
     if (info->split_k < 0 || info->split_k > SGEMM_MAX_SPLIT_K)
         return fail(SGEMM_E_CONFIG, "split_k = %d outside 0..%d", info->split_k, SGEMM_MAX_SPLIT_K);
+    // large launches may run the library's split-BF16 kernels (absent: never)
+    int split = 0;
+    CFG_TRY(toml_int(t, "split_bf16", &split, false, 0));
+    if (split < 0 || split > 1) return fail(SGEMM_E_CONFIG, "split_bf16 = %d outside 0..1", split);
+    *split_bf16 = split == 1;
     if (a_type || b_type || cd_type || scalar_type) return fail(SGEMM_E_CONFIG, "only FP32 (type 0) kernels are supported");
     info->trans_a = trans_a ? 1 : 0;
     info->trans_b = trans_b ? 1 : 0;
@@ -380,6 +386,9 @@ struct sgemm_handle {
     sgemm_handle* edge_cols = nullptr;        // strip of rows past the last tile row, of columns past the last
     int resident = 0;                         // work-groups of generated_gemm the device holds at once (0: unknown)
     hipStream_t own_stream = nullptr;         // created at sgemm_open; `stream` is it unless sgemm_set_stream
+    bool split_bf16 = false;                  // large launches may run the split-BF16 kernels (toml key split_bf16)
+    bool fixed_split = false;                 // sgemm_set_split_k fixed a count, sgemm_set_stream_k a mode: the
+    bool fixed_stream = false;                // handle's own kernels run
     std::vector<sgemm_handle*> edge_of;       // handles this one serves as an edge kernel (under g_edge_mutex)
 };
 
@@ -554,10 +563,66 @@ int decompose(const sgemm_handle* h, uint32_t m, uint32_t n, uint32_t k, uint32_
     return count;
 }
 
+SplitPlan split_plan(const sgemm_handle* h, uint32_t m, uint32_t n, uint32_t k, uint32_t lda, uint32_t ldb, uint32_t ldc,
+                     uint32_t ldd, float alpha, float beta) {
+    SplitPlan p;
+    if (!h->split_bf16 || h->fixed_split || h->fixed_stream || !bf16x6_launch || h->compute_units <= 0) return p;
+    if (k < bf16x6::kMinDepth || 2.0 * m * n * k < bf16x6::kMinFlops) return p;
+    if (std::max(std::max(lda, ldb), std::max(ldc, ldd)) >= bf16x6::kMaxLd) return p;
+    // alpha joins the unscaling factor 2^-32, which must not make it subnormal
+    if (alpha != 0.0f && std::fabs(alpha) < 1e-24f) return p;
+    const int cus = h->compute_units;
+    const bool reads_c = beta != 0.0f;
+    // the FP32 launch this one replaces: its time, and its sums' chains
+    Part parts[3];
+    const int count = decompose(h, m, n, k, lda, ldb, ldc, ldd, parts);
+    const Plan f = plan(h, parts[0].m, parts[0].n, k);
+    const uint64_t dk = (uint64_t)h->info.depth_k;
+    const uint64_t range = bf16x6::ceil_div(bf16x6::ceil_div(k, dk), f.splits) * dk;
+    double fp32 = bf16x6::fp32_time_us((uint64_t)h->info.tile_m, (uint64_t)h->info.tile_n, f.tiles * f.splits, range,
+                                       f.splits, f.sk_tiles != 0, parts[0].m, parts[0].n, k, reads_c, cus);
+    for (int q = 1; q < count; ++q) fp32 += bf16x6::strip_time_us(parts[q].m, parts[q].n, k);
+
+    double best = bf16x6::kMargin * fp32;
+    auto consider = [&](uint32_t pm, uint32_t pn, double strips) {
+        const bf16x6::Choice c = bf16x6::choose(pm, pn, k, h->info.trans_a != 0, reads_c, cus, f.splits);
+        if (c.tile < 0 || c.us + strips >= best) return;
+        best = c.us + strips;
+        p.tile = c.tile;
+        p.splits = c.splits;
+        p.m = pm;
+        p.n = pn;
+        p.partial_bytes = c.partial_bytes;
+        p.ticket_count = c.ticket_count;
+    };
+    consider(m, n, 0.0);
+    // thin strips past the last whole 128 rows or columns to the edge
+    // kernels: one row or column more would be a tile row or column more
+    const uint32_t me = h->edge_rows && m > 128 && m % 128 && m % 128 <= 16 ? m % 128 : 0u;
+    const uint32_t ne = h->edge_cols && n > 128 && n % 128 && n % 128 <= 16 ? n % 128 : 0u;
+    if (me || ne)
+        consider(m - me, n - ne, (me ? bf16x6::strip_time_us(me, n, k) : 0.0) +
+                                     (ne ? bf16x6::strip_time_us(m - me, ne, k) : 0.0));
+    return p;
+}
+
+int split_strips(const sgemm_handle* h, const SplitPlan& p, uint32_t m, uint32_t n, uint32_t lda, uint32_t ldb,
+                 uint32_t ldc, uint32_t ldd, Part out[2]) {
+    int count = 0;
+    const size_t mi = p.m, ni = p.n;
+    if (p.m < m)  // rows [mi, m) of every column
+        out[count++] = Part{h->edge_rows, m - p.m, n, h->info.trans_a ? mi * lda : mi, 0, mi, mi};
+    if (p.n < n)  // columns [ni, n) of rows [0, mi)
+        out[count++] = Part{h->edge_cols, p.m, n - p.n, 0, h->info.trans_b ? ni : ni * ldb, ni * ldc, ni * ldd};
+    return count;
+}
 
 hipStream_t stream(const sgemm_handle* h) { return h->stream; }
 
 int device(const sgemm_handle* h) { return h->device; }
+
+bool trans_a(const sgemm_handle* h) { return h->info.trans_a != 0; }
+bool trans_b(const sgemm_handle* h) { return h->info.trans_b != 0; }
 
 int set_error(int code, const char* message) { return fail(code, "%s", message); }
 
@@ -590,7 +655,8 @@ int sgemm_open(const char* co_path, const char* toml_path, sgemm_handle** out) {
     if (!co_path || !toml_path || !out) return fail(SGEMM_E_INVALID, "sgemm_open: null argument");
     *out = nullptr;
     sgemm_kernel_info info{};
-    int r = load_config(toml_path, &info);
+    bool split_bf16 = false;
+    int r = load_config(toml_path, &info, &split_bf16);
     if (r != SGEMM_OK) return r;
     {
         std::ifstream f(co_path, std::ios::binary);
@@ -601,6 +667,7 @@ int sgemm_open(const char* co_path, const char* toml_path, sgemm_handle** out) {
     if (e != hipSuccess || count == 0) return fail(SGEMM_E_NO_DEVICE, "no HIP device visible (%s)", hipGetErrorString(e));
     sgemm_handle* h = new sgemm_handle();
     h->info = info;
+    h->split_bf16 = split_bf16;
     hipError_t err = hipModuleLoad(&h->module, co_path);
     if (err != hipSuccess) {
         delete h;
@@ -645,7 +712,8 @@ int sgemm_open(const char* co_path, const char* toml_path, sgemm_handle** out) {
         if (!h->info.stream_k_groups) h->info.stream_k = 0;
         // the static scratch of sgemm_launch_noalloc on this device: looked
         // up here, so that no launch (maybe under graph capture) does it
-        const int sr = sgemm_internal::noalloc_prepare(dev);
+        int sr = sgemm_internal::noalloc_prepare(dev);
+        if (sr == SGEMM_OK && h->split_bf16 && sgemm_internal::bf16x6_prepare) sr = sgemm_internal::bf16x6_prepare();
         if (sr != SGEMM_OK) {
             sgemm_close(h);
             return sr;
@@ -745,6 +813,7 @@ int sgemm_set_split_k(sgemm_handle* h, int splits) {
     if (splits > h->info.split_k_max)
         return fail(SGEMM_E_CONFIG, "split count %d needs generated_gemm_splitk, absent from this code object", splits);
     h->info.split_k = splits;
+    h->fixed_split = splits != 0;
     return SGEMM_OK;
 }
 
@@ -765,13 +834,20 @@ int sgemm_workspace_size(const sgemm_handle* h, uint32_t m, uint32_t n, uint32_t
     if (!h || !bytes) return fail(SGEMM_E_INVALID, "sgemm_workspace_size: null argument");
     *bytes = 0;
     if (m && n) {
-        own_part(h, m, n, k, &m, &n);
-        const sgemm_internal::Plan p = sgemm_internal::plan(h, m, n, k);
+        uint32_t pm, pn;
+        own_part(h, m, n, k, &pm, &pn);
+        const sgemm_internal::Plan p = sgemm_internal::plan(h, pm, pn, k);
         size_t total = 0;
         if (p.partial_bytes && (__builtin_mul_overflow(p.ticket_count, (size_t)4, &total) ||
                                 __builtin_add_overflow(total, p.partial_bytes, &total)))
             total = SIZE_MAX;
         *bytes = p.partial_bytes ? total : 0;
+        // or the split-BF16 launch's (tight leading dimensions, alpha = 1)
+        const uint32_t lda = h->info.trans_a ? k : m, ldb = h->info.trans_b ? n : k;
+        const sgemm_internal::SplitPlan sp = sgemm_internal::split_plan(h, m, n, k, lda, ldb, m, m, 1.0f, 1.0f);
+        const sgemm_internal::SplitPlan sp0 = sgemm_internal::split_plan(h, m, n, k, lda, ldb, m, m, 1.0f, 0.0f);
+        for (const sgemm_internal::SplitPlan& q : {sp, sp0})
+            if (q.tile >= 0 && q.partial_bytes) *bytes = std::max(*bytes, q.partial_bytes + 4 * q.ticket_count);
     }
     return SGEMM_OK;
 }
@@ -782,6 +858,42 @@ int sgemm_set_stream_k(sgemm_handle* h, int mode) {
     if (mode && !h->info.stream_k_groups)
         return fail(SGEMM_E_CONFIG, "stream-K needs generated_gemm_streamk, absent from this code object");
     h->info.stream_k = mode;
+    h->fixed_stream = mode != 1;
+    return SGEMM_OK;
+}
+
+int sgemm_set_split_bf16(sgemm_handle* h, int mode) {
+    if (!h) return fail(SGEMM_E_INVALID, "sgemm_set_split_bf16: null handle");
+    if (mode < 0 || mode > 1) return fail(SGEMM_E_INVALID, "split-BF16 mode %d outside 0..1", mode);
+    if (mode && !sgemm_internal::bf16x6_launch)
+        return fail(SGEMM_E_CONFIG, "this build has no split-BF16 kernels");
+    if (mode && !h->split_bf16) {
+        // the handle's device loads the kernels now, so that no launch does
+        int cur = 0;
+        HIP_TRY(hipGetDevice(&cur));
+        if (cur != h->device) HIP_TRY(hipSetDevice(h->device));
+        const int r = sgemm_internal::bf16x6_prepare();
+        if (cur != h->device) (void)hipSetDevice(cur);
+        if (r != SGEMM_OK) return r;
+    }
+    h->split_bf16 = mode == 1;
+    return SGEMM_OK;
+}
+
+int sgemm_split_bf16_plan(const sgemm_handle* h, uint32_t m, uint32_t n, uint32_t k, uint32_t lda, uint32_t ldb,
+                          uint32_t ldc, uint32_t ldd, float alpha, float beta, int* tile_m, int* tile_n, int* splits,
+                          uint32_t* m_part, uint32_t* n_part) {
+    if (!h || !tile_m || !tile_n || !splits || !m_part || !n_part)
+        return fail(SGEMM_E_INVALID, "sgemm_split_bf16_plan: null argument");
+    const int r = sgemm_check_shape(h, m, n, k, lda, ldb, ldc, ldd);
+    if (r != SGEMM_OK) return r;
+    sgemm_internal::SplitPlan p;
+    if (m && n) p = sgemm_internal::split_plan(h, m, n, k, lda, ldb, ldc, ldd, alpha, beta);
+    *tile_m = p.tile < 0 ? 0 : bf16x6::kTiles[p.tile].m;
+    *tile_n = p.tile < 0 ? 0 : bf16x6::kTiles[p.tile].n;
+    *splits = p.tile < 0 ? 0 : (int)p.splits;
+    *m_part = p.tile < 0 ? 0 : p.m;
+    *n_part = p.tile < 0 ? 0 : p.n;
     return SGEMM_OK;
 }
 
@@ -834,36 +946,41 @@ int sgemm_memset(void* dptr, int value, size_t bytes) {
 
 namespace {
 
-// One part of a launch on `stream` with kernel handle `kh`: its split-K /
-// stream-K workspace is kh's own, grown on demand (both streams drained
-// first, fresh tickets zeroed on `stream`).
+// kh's own split-K / stream-K workspace, grown on demand to `ws_need` bytes of
+// partials and `tickets` tickets (both streams drained first, fresh tickets
+// zeroed on `stream`).
+int grow_workspace(sgemm_handle* kh, hipStream_t stream, size_t ws_need, size_t tickets) {
+    if (kh->ws_bytes >= ws_need && kh->ticket_count >= tickets) return SGEMM_OK;
+    HIP_TRY(hipStreamSynchronize(stream));
+    HIP_TRY(hipStreamSynchronize(kh->stream));
+    if (kh->ws_bytes < ws_need) {
+        if (kh->ws) HIP_TRY(hipFree(kh->ws));
+        kh->ws = nullptr;
+        kh->ws_bytes = 0;
+        HIP_TRY(hipMalloc(&kh->ws, ws_need));
+        kh->ws_bytes = ws_need;
+    }
+    if (kh->ticket_count < tickets) {
+        if (kh->tickets) HIP_TRY(hipFree(kh->tickets));
+        kh->tickets = nullptr;
+        kh->ticket_count = 0;
+        HIP_TRY(hipMalloc((void**)&kh->tickets, tickets * 4));
+        // ordered before the launch that follows on the same stream
+        HIP_TRY(hipMemsetAsync(kh->tickets, 0, tickets * 4, stream));
+        kh->ticket_count = tickets;
+    }
+    return SGEMM_OK;
+}
+
+// One part of a launch on `stream` with kernel handle `kh`.
 int launch_part(sgemm_handle* kh, hipStream_t stream, const float* dA, const float* dB, const float* dC, float* dD,
                 uint32_t m, uint32_t n, uint32_t k, uint32_t lda, uint32_t ldb, uint32_t ldc, uint32_t ldd, float alpha,
                 float beta) {
     const sgemm_internal::Plan p = sgemm_internal::plan(kh, m, n, k);
     if (!p.partial_bytes)
         return sgemm_internal::launch(kh, dA, dB, dC, dD, m, n, k, lda, ldb, ldc, ldd, alpha, beta, nullptr, stream);
-    const size_t ws_need = p.partial_bytes, tickets = p.ticket_count;
-    if (kh->ws_bytes < ws_need || kh->ticket_count < tickets) {
-        HIP_TRY(hipStreamSynchronize(stream));
-        HIP_TRY(hipStreamSynchronize(kh->stream));
-        if (kh->ws_bytes < ws_need) {
-            if (kh->ws) HIP_TRY(hipFree(kh->ws));
-            kh->ws = nullptr;
-            kh->ws_bytes = 0;
-            HIP_TRY(hipMalloc(&kh->ws, ws_need));
-            kh->ws_bytes = ws_need;
-        }
-        if (kh->ticket_count < tickets) {
-            if (kh->tickets) HIP_TRY(hipFree(kh->tickets));
-            kh->tickets = nullptr;
-            kh->ticket_count = 0;
-            HIP_TRY(hipMalloc((void**)&kh->tickets, tickets * 4));
-            // ordered before the launch below on the same stream
-            HIP_TRY(hipMemsetAsync(kh->tickets, 0, tickets * 4, stream));
-            kh->ticket_count = tickets;
-        }
-    }
+    const int r = grow_workspace(kh, stream, p.partial_bytes, p.ticket_count);
+    if (r != SGEMM_OK) return r;
     const sgemm_internal::Workspace ws{(float*)kh->ws, kh->ws_bytes, kh->tickets, kh->ticket_count};
     return sgemm_internal::launch(kh, dA, dB, dC, dD, m, n, k, lda, ldb, ldc, ldd, alpha, beta, &ws, stream);
 }
@@ -877,10 +994,19 @@ int sgemm_launch(sgemm_handle* h, const float* dA, const float* dB, const float*
     int r = sgemm_internal::check_launch(h, dA, dB, dC, dD, m, n, k, lda, ldb, ldc, ldd, beta);
     if (r != SGEMM_OK || m == 0 || n == 0) return r;
     sgemm_internal::Part parts[3];
-    const int count = sgemm_internal::decompose(h, m, n, k, lda, ldb, ldc, ldd, parts);
+    const sgemm_internal::SplitPlan sp = sgemm_internal::split_plan(h, m, n, k, lda, ldb, ldc, ldd, alpha, beta);
+    int count = sp.tile >= 0 ? sgemm_internal::split_strips(h, sp, m, n, lda, ldb, ldc, ldd, parts)
+                             : sgemm_internal::decompose(h, m, n, k, lda, ldb, ldc, ldd, parts);
     for (int q = 0; q < count; ++q) {
         const sgemm_internal::Part& pt = parts[q];
         if (pt.kh != h && (r = sgemm_check_shape(pt.kh, pt.m, pt.n, k, lda, ldb, ldc, ldd)) != SGEMM_OK) return r;
+    }
+    if (sp.tile >= 0) {
+        if ((r = grow_workspace(h, h->stream, sp.partial_bytes, sp.ticket_count)) != SGEMM_OK) return r;
+        r = sgemm_internal::bf16x6_launch(sp.tile, sp.splits, h->info.trans_a != 0, h->info.trans_b != 0, dA, dB, dC, dD,
+                                          sp.m, sp.n, k, lda, ldb, ldc, ldd, alpha, beta, (float*)h->ws, h->tickets,
+                                          h->stream);
+        if (r != SGEMM_OK) return r;
     }
     for (int q = 0; q < count; ++q) {
         const sgemm_internal::Part& pt = parts[q];

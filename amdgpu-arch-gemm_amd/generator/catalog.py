@@ -295,6 +295,13 @@ TWINS: Dict[Tuple[str, bool, bool], str] = {}
 NO_TWIN = {("mt256x128_a32_wg4x2_dk16_s3_occ4_plr2", True, False)}
 
 
+# The instances select() returns let the host library run large launches on
+# its split-BF16 kernels; the others always run their own (tuner points, the
+# variants that the tests compare with one another).
+for _name in list(CANDIDATES) + [nm for _, nm in PREFERRED]:
+    SOLUTIONS[_name][1].split_bf16 = 1
+
+
 def _add_twins() -> None:
     for name in EDGE_PAIR:
         cfg, opt = SOLUTIONS[name]

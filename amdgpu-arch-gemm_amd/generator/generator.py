@@ -158,6 +158,9 @@ class GemmOptimizations:
                        whole-tile rounds of work-groups for which the host
                        still picks stream-K on its own (0: no limit); tiles
                        whose stream-K kernel loses on long grids set it.
+    * ``split_bf16`` -- (host policy, written to the .toml) 1 lets the host
+                       library run large launches on its split-BF16 kernels
+                       instead of the code object's own (sgemm_set_split_bf16).
     """
 
     def __init__(
@@ -176,6 +179,7 @@ class GemmOptimizations:
         ws: Optional[int] = None,
         ws_pd: Optional[int] = None,
         ksplit: Optional[int] = None,
+        split_bf16: Optional[int] = None,
     ):
         self.level = level
         self.wgm = 1
@@ -191,6 +195,7 @@ class GemmOptimizations:
         self.ws = 0
         self.ws_pd = 2
         self.ksplit = 0
+        self.split_bf16 = 0
         self._setup_optimizations()
         if wgm is not None:
             self.wgm = wgm
@@ -218,6 +223,8 @@ class GemmOptimizations:
             self.ws_pd = ws_pd
         if ksplit is not None:
             self.ksplit = ksplit
+        if split_bf16 is not None:
+            self.split_bf16 = split_bf16
         if self.wgm < 1:
             raise RuntimeError(f"Invalid wgm: {self.wgm}")
         if self.map_k_idx and not _is_pow2(self.map_k_idx):
@@ -238,6 +245,8 @@ class GemmOptimizations:
             raise RuntimeError(f"Invalid wave specialisation ws={self.ws} ws_pd={self.ws_pd}")
         if self.ws and (self.split_k != 1 or self.stream_k):
             raise RuntimeError("wave specialisation (ws=1) builds no split-K or stream-K kernel")
+        if self.split_bf16 not in (0, 1):
+            raise RuntimeError(f"Invalid split_bf16 {self.split_bf16} (0 or 1)")
         if self.ksplit not in (0, 1):
             raise RuntimeError(f"Invalid in-group K split ksplit={self.ksplit}")
         if self.ksplit and (self.ws or self.split_k != 1 or self.stream_k or self.map_k_idx > 1):
@@ -264,6 +273,7 @@ class GemmOptimizations:
             "ws": int(self.ws),
             "ws_pd": int(self.ws_pd),
             "ksplit": int(self.ksplit),
+            "split_bf16": int(self.split_bf16),
         }
 
     def __repr__(self) -> str:
@@ -1090,7 +1100,7 @@ def build_kernel(output_folder: str, config: GemmSolutionConfig, opt: GemmOptimi
 def default_config(trans_a: bool = False, trans_b: bool = False) -> Tuple[GemmSolutionConfig, GemmOptimizations]:
     cfg = GemmSolutionConfig(DataType.FP32, DataType.FP32, DataType.FP32, DataType.FP32,
                              MFMA_32x32x2, (4, 2), (2, 4), 16, trans_a, trans_b, vmem_stage=2)
-    opt = GemmOptimizations(1, wgm=8, plr=3, gw=1, map_k_idx=0, xcd=8)
+    opt = GemmOptimizations(1, wgm=8, plr=3, gw=1, map_k_idx=0, xcd=8, split_bf16=1)
     return cfg, opt
 
 

@@ -66,6 +66,10 @@ SIGNATURES = {
     "sgemm_workspace_size": (_int, [_vp, _u32, _u32, _u32, ctypes.POINTER(ctypes.c_size_t)]),
     "sgemm_launch_splits": (_int, [_vp, _u32, _u32, _u32, ctypes.POINTER(_int)]),
     "sgemm_set_stream_k": (_int, [_vp, _int]),
+    "sgemm_set_split_bf16": (_int, [_vp, _int]),
+    "sgemm_split_bf16_plan": (_int, [_vp, _u32, _u32, _u32, _u32, _u32, _u32, _u32, _f32, _f32, ctypes.POINTER(_int),
+                                     ctypes.POINTER(_int), ctypes.POINTER(_int), ctypes.POINTER(_u32),
+                                     ctypes.POINTER(_u32)]),
     "sgemm_set_edge_kernel": (_int, [_vp, _vp]),
     "sgemm_set_edge_kernels": (_int, [_vp, _vp, _vp]),
     "sgemm_edge_interior": (_int, [_vp, _u32, _u32, _u32, ctypes.POINTER(_u32), ctypes.POINTER(_u32)]),
@@ -276,6 +280,21 @@ class Kernel:
         """0: never stream-K; 1: when a partial last round of work-groups costs >= 3%; 2: whenever tiles > groups."""
         _check("sgemm_set_stream_k", load_library().sgemm_set_stream_k(self.handle, int(mode)))
         self._refresh_info()
+
+    def set_split_bf16(self, mode: int):
+        """0: this instance's own FP32 kernels only; 1: the split-BF16 kernels wherever they are expected to be faster."""
+        _check("sgemm_set_split_bf16", load_library().sgemm_set_split_bf16(self.handle, int(mode)))
+
+    def split_bf16_plan(self, m, n, k, alpha=1.0, beta=0.0, lda=None, ldb=None, ldc=None, ldd=None) -> Optional[dict]:
+        """Tile, K ranges and part (m, n) of the split-BF16 kernel a launch runs on; None: this instance's own kernels."""
+        da, db = self.default_lds(m, n, k)
+        tm, tn, sp, pm, pn = _int(), _int(), _int(), _u32(), _u32()
+        _check("sgemm_split_bf16_plan", load_library().sgemm_split_bf16_plan(
+            self.handle, m, n, k, lda or da, ldb or db, ldc or m, ldd or m, alpha, beta, ctypes.byref(tm),
+            ctypes.byref(tn), ctypes.byref(sp), ctypes.byref(pm), ctypes.byref(pn)))
+        if not tm.value:
+            return None
+        return {"tile": (tm.value, tn.value), "splits": sp.value, "part": (int(pm.value), int(pn.value))}
 
     def set_edge_kernel(self, edge: Optional["Kernel"]):
         """One small-tile kernel for both thin edge strips (None detaches); it must stay open while attached."""

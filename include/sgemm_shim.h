@@ -141,8 +141,9 @@ int sgemm_check_shape(const sgemm_handle* h, uint32_t m, uint32_t n, uint32_t k,
 int sgemm_set_split_k(sgemm_handle* h, int splits);
 
 /* Device bytes the handle's workspace needs for an m x n x k launch with its
- * current split and stream-K settings (0 when the launch needs none; h's own
- * part: the interior when edge kernels take strips).  No
+ * current settings (0 when the launch needs none; h's own
+ * part: the interior when edge kernels take strips; the larger of h's own
+ * kernels' need and a split-BF16 launch's).  No
  * counterpart in the reference (its kernel needs no workspace). */
 int sgemm_workspace_size(const sgemm_handle* h, uint32_t m, uint32_t n, uint32_t k, size_t* bytes);
 
@@ -165,6 +166,31 @@ int sgemm_launch_splits(const sgemm_handle* h, uint32_t m, uint32_t n, uint32_t 
  * counterpart in the reference (its grid is one work-group per tile,
  * generator_runner.cpp:127-131). */
 int sgemm_set_stream_k(sgemm_handle* h, int mode);
+
+/* Sets whether later launches of h may run the library's split-BF16 kernels in
+ * place of h's own: 0 never, 1 (the default of instances whose .toml has
+ * split_bf16 = 1) wherever a time model of both expects them to be at least 5%
+ * faster (from about 2 GFLOP: cubes past 1280, 16384 x 128 x 4096, ...).
+ * Each FP32 value of A and B is split into three BF16 terms (exactly: 24 bits)
+ * and six of their nine products are summed in FP32 on the BF16 matrix cores;
+ * against 64 bits the result is no further off than the FP32 kernels'.  NaN,
+ * Inf, overflow and subnormals give what the FP32 kernels give (a tile that
+ * meets a value out of range is run again with FP32 MFMAs, at their speed).
+ * A launch runs on h's own kernels all the same while h has a fixed K split
+ * (sgemm_set_split_k above 0) or stream-K mode (sgemm_set_stream_k 0 or 2),
+ * for a leading dimension of 2^21 or more, and for 0 < |alpha| < 1e-24.
+ * sgemm_launch_splits, sgemm_stream_k_tiles and sgemm_edge_interior describe
+ * h's own kernels.  SGEMM_E_INVALID outside 0..1.  No counterpart in the
+ * reference, whose kernels multiply in FP32. */
+int sgemm_set_split_bf16(sgemm_handle* h, int mode);
+
+/* How a launch with these arguments runs with h's current settings: the tile
+ * and K ranges of the split-BF16 kernel and the rows and columns it takes
+ * (all of them, or the whole tiles when h's edge kernels take a thin strip),
+ * or zeros when h's own kernels run.  No counterpart in the reference. */
+int sgemm_split_bf16_plan(const sgemm_handle* h, uint32_t m, uint32_t n, uint32_t k, uint32_t lda, uint32_t ldb,
+                          uint32_t ldc, uint32_t ldd, float alpha, float beta, int* tile_m, int* tile_n, int* splits,
+                          uint32_t* m_part, uint32_t* n_part);
 
 /* Attaches two other loaded kernels with the same trans_a / trans_b that
  * later launches of h use for thin edge strips: `rows` (tile_m below h's)
