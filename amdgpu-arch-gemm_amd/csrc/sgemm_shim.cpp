@@ -753,6 +753,10 @@ void sgemm_close(sgemm_handle* h) {
     }
     if (h->stream) (void)hipStreamSynchronize(h->stream);
     if (h->own_stream && h->own_stream != h->stream) (void)hipStreamSynchronize(h->own_stream);
+    if (sgemm_internal::noalloc_forget && h->own_stream) {
+        sgemm_internal::noalloc_forget(h->device, h->stream);
+        sgemm_internal::noalloc_forget(h->device, h->own_stream);
+    }
     if (h->ev_start) (void)hipEventDestroy(h->ev_start);
     if (h->ev_stop) (void)hipEventDestroy(h->ev_stop);
     if (h->own_stream) (void)hipStreamDestroy(h->own_stream);
@@ -1136,6 +1140,7 @@ int sgemm_set_stream(sgemm_handle* h, void* stream) {
         if (cs != hipStreamCaptureStatusNone)
             return fail(SGEMM_E_INVALID, "sgemm_set_stream: the handle's current stream is capturing");
         HIP_TRY(hipStreamSynchronize(h->stream));
+        if (sgemm_internal::noalloc_forget) sgemm_internal::noalloc_forget(h->device, h->stream);
         h->stream = next;
     }
     return SGEMM_OK;
