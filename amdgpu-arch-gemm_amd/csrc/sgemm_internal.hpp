@@ -4,6 +4,7 @@
 #pragma once
 
 #include "sgemm_shim.h"
+#include "thin_plan.hpp"
 
 #include <hip/hip_runtime_api.h>
 
@@ -88,9 +89,19 @@ SGEMM_INTERNAL __attribute__((weak)) int bf16x6_launch(int tile, uint32_t splits
                                                        uint32_t m, uint32_t n, uint32_t k, uint32_t lda, uint32_t ldb,
                                                        uint32_t ldc, uint32_t ldd, float alpha, float beta,
                                                        float* partials, uint32_t* tickets, hipStream_t stream);
+// Whether and how a launch runs on the thin kernel (thin_plan.hpp); such a
+// launch has no split plan.
+SGEMM_INTERNAL thin::Shape thin_shape(const sgemm_handle* h, uint32_t m, uint32_t n, uint32_t k, uint32_t lda,
+                                      uint32_t ldb);
+// Enqueues one checked launch of the thin kernel.  Weak, as bf16x6_launch.
+SGEMM_INTERNAL __attribute__((weak)) int thin_launch(const thin::Shape& t, bool trans_a, bool trans_b, const float* dA,
+                                                     const float* dB, const float* dC, float* dD, uint32_t m, uint32_t n,
+                                                     uint32_t k, uint32_t lda, uint32_t ldb, uint32_t ldc, uint32_t ldd,
+                                                     float alpha, float beta, hipStream_t stream);
 // Loads the split-BF16 kernels on the current device, so that no launch
 // (maybe under graph capture) does.
 SGEMM_INTERNAL __attribute__((weak)) int bf16x6_prepare();
+SGEMM_INTERNAL __attribute__((weak)) int thin_prepare();   // the same for the thin kernels
 
 // Looks up the device address of sgemm_launch_noalloc's static scratch on
 // device `dev` (once per device; later calls return at once).  sgemm_open

@@ -184,6 +184,10 @@ extern "C" int sgemm_launch_noalloc(sgemm_handle* h, const float* dA, const floa
     int r = sgemm_internal::check_launch(h, dA, dB, dC, dD, m, n, k, lda, ldb, ldc, ldd, beta);
     if (r != SGEMM_OK || m == 0 || n == 0) return r;
     hipStream_t s = sgemm_internal::stream(h);
+    const thin::Shape ts = sgemm_internal::thin_shape(h, m, n, k, lda, ldb);
+    if (ts.on)
+        return sgemm_internal::thin_launch(ts, sgemm_internal::trans_a(h), sgemm_internal::trans_b(h), dA, dB, dC, dD, m,
+                                           n, k, lda, ldb, ldc, ldd, alpha, beta, s);
     sgemm_internal::Part parts[3];
     // the split-BF16 plan never needs more than the scratch
     const sgemm_internal::SplitPlan sp = sgemm_internal::split_plan(h, m, n, k, lda, ldb, ldc, ldd, alpha, beta);

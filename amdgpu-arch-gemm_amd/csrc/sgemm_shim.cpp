@@ -563,10 +563,16 @@ int decompose(const sgemm_handle* h, uint32_t m, uint32_t n, uint32_t k, uint32_
     return count;
 }
 
+thin::Shape thin_shape(const sgemm_handle* h, uint32_t m, uint32_t n, uint32_t k, uint32_t lda, uint32_t ldb) {
+    if (!h->split_bf16 || h->fixed_split || h->fixed_stream || !thin_launch) return thin::Shape();
+    return thin::choose(m, n, k, lda, ldb, h->info.trans_a != 0, h->info.trans_b != 0);
+}
+
 SplitPlan split_plan(const sgemm_handle* h, uint32_t m, uint32_t n, uint32_t k, uint32_t lda, uint32_t ldb, uint32_t ldc,
                      uint32_t ldd, float alpha, float beta) {
     SplitPlan p;
     if (!h->split_bf16 || h->fixed_split || h->fixed_stream || !bf16x6_launch || h->compute_units <= 0) return p;
+    if (thin_shape(h, m, n, k, lda, ldb).on) return p;
     if (k < bf16x6::kMinDepth || 2.0 * m * n * k < bf16x6::kMinFlops) return p;
     if (std::max(std::max(lda, ldb), std::max(ldc, ldd)) >= bf16x6::kMaxLd) return p;
     // alpha joins the unscaling factor 2^-32, which must not make it subnormal
@@ -714,6 +720,7 @@ int sgemm_open(const char* co_path, const char* toml_path, sgemm_handle** out) {
         // up here, so that no launch (maybe under graph capture) does it
         int sr = sgemm_internal::noalloc_prepare(dev);
         if (sr == SGEMM_OK && h->split_bf16 && sgemm_internal::bf16x6_prepare) sr = sgemm_internal::bf16x6_prepare();
+        if (sr == SGEMM_OK && h->split_bf16 && sgemm_internal::thin_prepare) sr = sgemm_internal::thin_prepare();
         if (sr != SGEMM_OK) {
             sgemm_close(h);
             return sr;
@@ -876,7 +883,8 @@ int sgemm_set_split_bf16(sgemm_handle* h, int mode) {
         int cur = 0;
         HIP_TRY(hipGetDevice(&cur));
         if (cur != h->device) HIP_TRY(hipSetDevice(h->device));
-        const int r = sgemm_internal::bf16x6_prepare();
+        int r = sgemm_internal::bf16x6_prepare();
+        if (r == SGEMM_OK && sgemm_internal::thin_prepare) r = sgemm_internal::thin_prepare();
         if (cur != h->device) (void)hipSetDevice(cur);
         if (r != SGEMM_OK) return r;
     }
@@ -997,6 +1005,10 @@ int sgemm_launch(sgemm_handle* h, const float* dA, const float* dB, const float*
     if (!h) return fail(SGEMM_E_INVALID, "sgemm_launch: null handle");
     int r = sgemm_internal::check_launch(h, dA, dB, dC, dD, m, n, k, lda, ldb, ldc, ldd, beta);
     if (r != SGEMM_OK || m == 0 || n == 0) return r;
+    const thin::Shape ts = sgemm_internal::thin_shape(h, m, n, k, lda, ldb);
+    if (ts.on)
+        return sgemm_internal::thin_launch(ts, h->info.trans_a != 0, h->info.trans_b != 0, dA, dB, dC, dD, m, n, k, lda,
+                                           ldb, ldc, ldd, alpha, beta, h->stream);
     sgemm_internal::Part parts[3];
     const sgemm_internal::SplitPlan sp = sgemm_internal::split_plan(h, m, n, k, lda, ldb, ldc, ldd, alpha, beta);
     int count = sp.tile >= 0 ? sgemm_internal::split_strips(h, sp, m, n, lda, ldb, ldc, ldd, parts)

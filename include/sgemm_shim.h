@@ -176,6 +176,8 @@ int sgemm_set_stream_k(sgemm_handle* h, int mode);
  * against 64 bits the result is no further off than the FP32 kernels'.  NaN,
  * Inf, overflow and subnormals give what the FP32 kernels give (a tile that
  * meets a value out of range is run again with FP32 MFMAs, at their speed).
+ * Mode 1 also lets a launch with m or n at most 16 run on a kernel that
+ * streams the large operand (FP32 MFMAs, no workspace), where that is faster.
  * A launch runs on h's own kernels all the same while h has a fixed K split
  * (sgemm_set_split_k above 0) or stream-K mode (sgemm_set_stream_k 0 or 2),
  * for a leading dimension of 2^21 or more, and for 0 < |alpha| < 1e-24.
@@ -187,7 +189,7 @@ int sgemm_set_split_bf16(sgemm_handle* h, int mode);
 /* How a launch with these arguments runs with h's current settings: the tile
  * and K ranges of the split-BF16 kernel and the rows and columns it takes
  * (all of them, or the whole tiles when h's edge kernels take a thin strip),
- * or zeros when h's own kernels run.  No counterpart in the reference. */
+ * or zeros when h's own kernels or the thin one run.  No counterpart in the reference. */
 int sgemm_split_bf16_plan(const sgemm_handle* h, uint32_t m, uint32_t n, uint32_t k, uint32_t lda, uint32_t ldb,
                           uint32_t ldc, uint32_t ldd, float alpha, float beta, int* tile_m, int* tile_n, int* splits,
                           uint32_t* m_part, uint32_t* n_part);
