@@ -221,6 +221,12 @@ def main():
     m, n, k, seed, dist = WORKLOADS[args.workload]
     co, toml = catalog.paths(args.kernel)
     os.makedirs(args.out, exist_ok=True)
+    # the instance itself is profiled, not the library's split-BF16 kernels
+    with open(toml) as f:
+        text = f.read().replace("split_bf16 = 1", "split_bf16 = 0")
+    toml = os.path.join(args.out, "fp32.toml")
+    with open(toml, "w") as f:
+        f.write(text)
     warmup = args.warmup if args.warmup is not None else WARMUP[args.workload]
     runner = [RUNNER, co, toml, str(m), str(n), str(k), str(warmup), str(args.runs), "0", str(seed), str(dist), "1", "0"]
     probe = [PROBE, str(PROBE_BYTES), "3"]

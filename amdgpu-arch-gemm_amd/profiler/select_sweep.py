@@ -44,6 +44,7 @@ def main() -> int:
     kerns = {}
     for c in cands:
         kern = S.Kernel(*catalog.paths(c))
+        kern.set_split_bf16(0)   # the instance itself is timed
         if kern.info.split_k_max > 1:
             kern.set_split_k(0)
         kerns[c] = kern

@@ -21,6 +21,13 @@ both float32 results with the float64 product of the same inputs.  A second,
 separately labelled CPU figure (cpu_baseline.parallel) runs the same loop over
 columns on up to 16 host threads (about 5 s).
 
+Launches of this size run on the library's split-BF16 kernels (FP32 operands,
+each split exactly into three BF16 terms, six products summed in FP32; no
+further from float64 than the FP32 kernels: parity.gpu_vs_f64): config.split_bf16
+is their plan, null when the instance's own FP32 kernel ran, and roofline.peak
+is that of the units that ran.  --split-bf16 0, --kernel, --split-k and
+--stream-k time the FP32 kernel.
+
 --layout tn / nt / tt stores A (k x m) and/or B (n x k) transposed and runs
 the instance catalog.select picks for that layout (op(A) = A^T, op(B) = B^T);
 the CPU baseline multiplies the transposed-back operands.
@@ -44,6 +51,9 @@ import numpy as np  # noqa: E402
 from generator import catalog  # noqa: E402
 from shim import sgemm_shim as S  # noqa: E402
 
+# six BF16 products to one FP32 product on the split-BF16 kernels, at the 2516.6
+# TFLOP/s dense BF16 peak (256 CU x 4096 FLOP/clk x 2.4 GHz)
+SPLIT_BF16_PEAK_TFLOPS = 2516.6 / 6.0
 FP32_MFMA_PEAK_TFLOPS = 157.3  # MI355X dense FP32 matrix peak (256 CU x 256 FLOP/clk x 2.4 GHz)
 HBM_PEAK_GBS = 8000.0
 
@@ -169,6 +179,9 @@ def main():
                     help="K ranges per output tile (0 = per problem; default: the instance's own setting)")
     ap.add_argument("--stream-k", type=int, default=None,
                     help="stream-K mode (0 off, 1 auto, 2 forced; default: the instance's own setting)")
+    ap.add_argument("--split-bf16", type=int, default=None, choices=[0, 1],
+                    help="0: the instance's own FP32 kernel; 1: the split-BF16 kernels where they are faster "
+                         "(default: the instance's own setting, 0 with --kernel)")
     ap.add_argument("--no-edge", action="store_true", help="do not attach the catalog's edge kernel")
     ap.add_argument("--layout", default="nn", choices=["nn", "tn", "nt", "tt"],
                     help="operand layout: t stores A (k x m) or B (n x k) transposed")
@@ -205,9 +218,16 @@ def main():
         kern.set_split_k(args.split_k)
     if args.stream_k is not None:
         kern.set_stream_k(args.stream_k)
+    if args.split_bf16 is not None or args.kernel:
+        kern.set_split_bf16(args.split_bf16 or 0)
     splits = kern.launch_splits(m, n, k)
     sk_tiles = kern.stream_k_tiles(m, n, k) if kern.info.stream_k_groups else 0
-    log(f"K ranges per output tile: {splits}; stream-K tiles: {sk_tiles}")
+    plan = kern.split_bf16_plan(m, n, k)
+    if plan:
+        splits, sk_tiles = plan["splits"], 0
+        interior = plan["part"]
+    peak = SPLIT_BF16_PEAK_TFLOPS if plan else FP32_MFMA_PEAK_TFLOPS
+    log(f"split-BF16 plan: {plan}; K ranges per output tile: {splits}; stream-K tiles: {sk_tiles}")
     dA, dB = S.DeviceBuffer.from_array(A), S.DeviceBuffer.from_array(B)
     dD = S.DeviceBuffer(m * n * 4)
     dD.zero()
@@ -248,7 +268,7 @@ def main():
     # A, B read once and D written once; a split launch also writes and
     # reads its partials (4 bytes per output per K range), not counted here
     alg_bytes = 4.0 * (m * k + k * n + m * n)
-    traffic = read_traffic(name, args.workload)
+    traffic = read_traffic("split_bf16_%dx%d" % plan["tile"] if plan else name, args.workload)
     line = {
         "metric": (HEADLINE_METRIC if (args.workload, args.layout) == ("cfg3", "nn")
                    else f"FP32 SGEMM TFLOP/s at {m}x{n}x{k} {args.layout.upper()}"),
@@ -269,6 +289,7 @@ def main():
             "dist": "uniform[-1,1)" if dist == S.SGEMM_DIST_UNIFORM else "normal(0,1)",
             "alpha": 1.0, "beta": 0.0,
             "kernel": name,
+            "split_bf16": plan,
             "split_k": splits,
             "stream_k_tiles": sk_tiles,
             "edge_kernels": list(catalog.EDGE_KERNEL[name]) if interior != (m, n) else None,
@@ -279,9 +300,9 @@ def main():
         "roofline": {
             "bound": "mfma",
             "achieved": round(achieved, 3),
-            "peak": FP32_MFMA_PEAK_TFLOPS,
+            "peak": round(peak, 1),
             "unit": "TFLOP/s",
-            "frac": round(achieved / FP32_MFMA_PEAK_TFLOPS, 4),
+            "frac": round(achieved / round(peak, 1), 4),
             "traffic": traffic,
             "kernel_ms_mean": round(kernel_ms, 5),
             "kernel_ms_median": round(median_ms, 5),

@@ -169,7 +169,7 @@ int sgemm_set_stream_k(sgemm_handle* h, int mode);
 
 /* Sets whether later launches of h may run the library's split-BF16 kernels in
  * place of h's own: 0 never, 1 (the default of instances whose .toml has
- * split_bf16 = 1) wherever a time model of both expects them to be at least 5%
+ * split_bf16 = 1) wherever a time model of both expects them to be at least 7%
  * faster (from about 2 GFLOP: cubes past 1280, 16384 x 128 x 4096, ...).
  * Each FP32 value of A and B is split into three BF16 terms (exactly: 24 bits)
  * and six of their nine products are summed in FP32 on the BF16 matrix cores;
