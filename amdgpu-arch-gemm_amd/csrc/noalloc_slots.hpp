@@ -1,0 +1,102 @@
+// Which part of sgemm_launch_noalloc's scratch a call works in, and what it
+// waits for first.  Host only; no HIP: `Streams` is the stream runtime, so that
+// the rules run against a model of it in a test.
+//
+// The scratch is cut into kSlots slots, each owned by the stream whose calls
+// used it last.  A call that fits a slot takes its stream's own one, a free one,
+// or the one longest unused; a larger call takes them all.  Work of another
+// owner is waited for on the device, by an event recorded on its stream when the
+// slot is taken over: a call on a slot that its stream owns costs nothing.
+//
+// A stream that is capturing cannot be recorded on (the event would join its
+// graph) and is taken for idle.
+//
+// Captured calls run when their graph is replayed, which is the caller's to
+// order against everything else on the device: they begin at the first slot and
+// leave the owners alone.
+#pragma once
+
+#include <cstddef>
+#include <cstdint>
+
+namespace noalloc {
+
+constexpr int kSlots = 8;
+constexpr int kBusy = -1000;   // no scratch for this call now
+
+// Streams:
+//   typedef ... Stream;
+//   bool capturing(Stream s, uint64_t* id)   whether s is capturing, in which capture
+//   int order(Stream before, Stream after)   later work of `after` waits for the work enqueued on `before`
+// and every int is 0 on success.
+template <class Streams> class Slots {
+  public:
+    typedef typename Streams::Stream Stream;
+
+    // Takes one slot (all: every slot) for the call that is enqueued on `s`
+    // next.  *first: its slot; *fresh: its tickets may be another stream's;
+    // *captured: the call is part of a capture.
+    int take(Streams& streams, Stream s, bool all, int* first, bool* fresh, bool* captured) {
+        uint64_t id = 0;
+        *first = 0;
+        *fresh = *captured = streams.capturing(s, &id);
+        if (*captured) return 0;
+        auto own = [&](const Slot& t) { return t.state == kOwned && t.owner == s; };
+        if (!all)
+            for (Slot& t : slots_)
+                if (own(t)) {
+                    *first = (int)(&t - slots_);
+                    t.used = ++calls_;
+                    return 0;
+                }
+        uint64_t other = 0;
+        if (!all) {
+            auto rank = [&](int q) { return slots_[q].state == kFree ? 1 : 2; };
+            for (int q = 1; q < kSlots; ++q)
+                if (rank(q) < rank(*first) || (rank(q) == rank(*first) && slots_[q].used < slots_[*first].used)) *first = q;
+        }
+        const int end = all ? kSlots : *first + 1;
+        for (int q = *first; q < end; ++q) {
+            Slot& t = slots_[q];
+            if (!own(t)) {
+                *fresh = true;
+                bool waited = t.state == kFree || streams.capturing(t.owner, &other);
+                for (int p = *first; p < q && !waited; ++p) waited = t.state == kOwned && was_[p] && old_[p] == t.owner;
+                if (!waited) {
+                    const int e = streams.order(t.owner, s);
+                    if (e) return e;
+                }
+            }
+            was_[q] = t.state == kOwned;
+            old_[q] = t.owner;
+        }
+        for (int q = *first; q < end; ++q) {
+            slots_[q].state = kOwned;
+            slots_[q].owner = s;
+            slots_[q].used = calls_ + 1;
+        }
+        ++calls_;
+        return 0;
+    }
+
+    // `s`, whose work has ended, is about to be destroyed, or a handle leaves it.
+    int forget(Streams&, Stream s) {
+        for (Slot& t : slots_)
+            if (t.state == kOwned && t.owner == s) t.state = kFree;
+        return 0;
+    }
+
+  private:
+    enum State { kFree, kOwned };
+    struct Slot {
+        State state = kFree;
+        Stream owner = Stream();
+        uint64_t used = 0;
+    };
+    Slot slots_[kSlots];
+    bool was_[kSlots];
+    Stream old_[kSlots];
+    uint64_t calls_ = 0;
+};
+
+}  // namespace noalloc

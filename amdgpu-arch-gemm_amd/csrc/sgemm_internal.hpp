@@ -44,10 +44,10 @@ SGEMM_INTERNAL int check_launch(const sgemm_handle* h, const float* dA, const fl
 
 // Enqueues one checked launch of h's kernels on `stream`.  A split-K or
 // stream-K launch uses `ws` (its sizes must cover plan()'s needs); a plain one
-// ignores it.
+// ignores it.  whole_k: a plain one whatever the plan says.
 SGEMM_INTERNAL int launch(sgemm_handle* h, const float* dA, const float* dB, const float* dC, float* dD, uint32_t m,
                           uint32_t n, uint32_t k, uint32_t lda, uint32_t ldb, uint32_t ldc, uint32_t ldd, float alpha,
-                          float beta, const Workspace* ws, hipStream_t stream);
+                          float beta, const Workspace* ws, hipStream_t stream, bool whole_k = false);
 
 // One part of a launch: kernel handle `kh` on an m x n block whose A, B, C,
 // D start `*_off` floats into the caller's matrices.

@@ -15,6 +15,7 @@
 // reads the stored pointer.
 
 #include "bf16x6_plan.hpp"
+#include "noalloc_slots.hpp"
 #include "sgemm_internal.hpp"
 
 #include <hip/hip_runtime.h>
@@ -46,31 +47,44 @@ constexpr int kMaxDevices = 64;
 std::mutex g_mutex;
 void* g_scratch[kMaxDevices];  // device address of each device's `scratch`, null until looked up
 
-// Who uses each device's scratch.  It is cut into kSlots slots of partials and
-// tickets; a launch that fits one takes the slot its stream owns, or a free
-// one, or -- every other stream's call on it waited for, by an event recorded on
-// that stream at that moment -- the one longest unused; a larger launch takes
-// them all.  So calls of up to kSlots streams run side by side, and as every
-// launch leaves its tickets zero and the stream orders a slot's launches, a
-// call on the slot its stream owns needs no clearing kernel of its own
-// (333 x 129 x 517 in 4 K ranges: 7.7 -> 4.9 us; one slot for all with a wait
-// between streams took 18.6 us where three streams took turns).
+// Who uses each device's scratch: noalloc_slots.hpp.  A slot holds an eighth of
+// the partials and tickets, so calls of up to eight streams run side by side;
+// every launch leaves its tickets zero and a slot's launches are ordered by
+// its stream, so a call on the slot its stream owns needs no clearing kernel of
+// its own (333 x 129 x 517 in 4 K ranges: 7.7 -> 4.9 us; one slot for all with a
+// wait between streams took 18.6 us where three streams took turns).
 // Captured calls, whose replays are not seen here, clear their tickets, and
-// so does every call on a device once one has been captured.  Owners are
-// streams of open handles (noalloc_forget).
-constexpr int kSlots = 8;
-constexpr size_t kSlotBytes = (size_t)SGEMM_NOALLOC_PARTIAL_BYTES / kSlots;
-constexpr size_t kSlotTickets = (size_t)SGEMM_NOALLOC_MAX_TILES / kSlots;
-struct Slot {
-    hipStream_t owner = nullptr;
-    bool owned = false;
-    uint64_t used = 0;
+// so does every call on a device once one has been captured.
+constexpr size_t kSlotBytes = (size_t)SGEMM_NOALLOC_PARTIAL_BYTES / noalloc::kSlots;
+constexpr size_t kSlotTickets = (size_t)SGEMM_NOALLOC_MAX_TILES / noalloc::kSlots;
+
+// The runtime that noalloc::Slots speaks to, on one device.
+struct HipStreams {
+    typedef hipStream_t Stream;
+    hipEvent_t moment = nullptr;                 // recorded and waited for within one order()
+
+    bool capturing(hipStream_t s, uint64_t* id) {
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        unsigned long long n = 0;
+        // an error: the null stream while another one captures
+        const bool on = hipStreamGetCaptureInfo(s, &cs, &n) != hipSuccess || cs != hipStreamCaptureStatusNone;
+        *id = n;
+        return on;
+    }
+    int order(hipStream_t before, hipStream_t after) {
+        hipError_t e = hipEventRecord(moment, before);
+        if (e != hipSuccess) return (int)e;
+        return (int)hipStreamWaitEvent(after, moment, 0);
+    }
+    hipError_t create() {
+        return moment ? hipSuccess : hipEventCreateWithFlags(&moment, hipEventDisableTiming);
+    }
 };
+
 struct Use {
-    Slot slots[kSlots];
-    uint64_t calls = 0;
+    noalloc::Slots<HipStreams> slots;
+    HipStreams streams;
     bool captured = false;
-    hipEvent_t event = nullptr;
 };
 std::mutex g_use_mutex;
 Use g_use[kMaxDevices];
@@ -86,7 +100,7 @@ int scratch_address(int dev, void** out) {
         if (e == hipSuccess && cur != dev) e = hipSetDevice(dev);
         void* p = nullptr;
         if (e == hipSuccess) e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
-        if (e == hipSuccess) e = hipEventCreateWithFlags(&g_use[dev].event, hipEventDisableTiming);
+        if (e == hipSuccess) e = g_use[dev].streams.create();
         if (cur != dev) (void)hipSetDevice(cur);
         if (e != hipSuccess || !p) {
             char msg[256];
@@ -100,67 +114,43 @@ int scratch_address(int dev, void** out) {
     return SGEMM_OK;
 }
 
-bool is_capturing(hipStream_t s) {
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    return hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone;
-}
-
 int launch_failed(hipError_t e, const char* what) {
     char msg[256];
     snprintf(msg, sizeof(msg), "%s failed: %s (%d)", what, hipGetErrorString(e), (int)e);
     return sgemm_internal::set_error((int)e, msg);
 }
 
+// One call's part of a device's scratch.
+struct Scratch {
+    float* partials = nullptr;
+    uint32_t* tickets = nullptr;
+    bool all = false;
+    int first = 0;
+};
+
 // Partials (`bytes`) and tickets (`count`, zero) on h's device for the launch
-// that the caller enqueues on `s` next, with `lock` still held.
+// that the caller enqueues on `s` next, with `lock` still held.  noalloc::kBusy: none now.
 int take_scratch(const sgemm_handle* h, size_t bytes, size_t count, hipStream_t s, std::unique_lock<std::mutex>& lock,
-                 float** partials, uint32_t** tickets) {
+                 Scratch* out) {
     const int dev = sgemm_internal::device(h);
     void* base = nullptr;
     const int r = scratch_address(dev, &base);
     if (r != SGEMM_OK) return r;
     if (!lock.owns_lock()) lock.lock();
     Use& u = g_use[dev];
-    const bool capturing = is_capturing(s);
-    u.captured = u.captured || capturing;
-    bool clear = u.captured;
-    // takes slot q for s; waits for another owner's launches
-    auto take = [&](int q) -> hipError_t {
-        Slot& t = u.slots[q];
-        hipError_t e = hipSuccess;
-        if (!t.owned || t.owner != s) {
-            clear = true;
-            if (t.owned && !capturing && !is_capturing(t.owner)) {
-                e = hipEventRecord(u.event, t.owner);
-                if (e == hipSuccess) e = hipStreamWaitEvent(s, u.event, 0);
-            }
-            t.owned = true;
-            t.owner = s;
-        }
-        t.used = ++u.calls;
-        return e;
-    };
-    int first = 0;
-    hipError_t e = hipSuccess;
-    if (bytes <= kSlotBytes && count <= kSlotTickets) {
-        // the stream's own slot, else a free one, else the one longest unused
-        auto rank = [&](const Slot& t) { return t.owned && t.owner == s ? 0 : (t.owned ? 2 : 1); };
-        for (int q = 1; q < kSlots; ++q) {
-            const Slot &x = u.slots[q], &y = u.slots[first];
-            if (rank(x) < rank(y) || (rank(x) == rank(y) && x.used < y.used)) first = q;
-        }
-        e = take(first);
-    } else {
-        for (int q = 0; q < kSlots && e == hipSuccess; ++q) e = take(q);
-    }
-    if (e != hipSuccess) return launch_failed(e, "ordering two streams' calls");
+    out->all = bytes > kSlotBytes || count > kSlotTickets;
+    bool fresh = false, captured = false;
+    int e = u.slots.take(u.streams, s, out->all, &out->first, &fresh, &captured);
+    u.captured = u.captured || captured;
+    if (e == noalloc::kBusy) return e;
+    if (e) return launch_failed((hipError_t)e, "ordering two streams' calls");
     unsigned char* const bytes0 = static_cast<unsigned char*>(base);
-    *partials = reinterpret_cast<float*>(bytes0 + (size_t)first * kSlotBytes);
-    *tickets = reinterpret_cast<uint32_t*>(bytes0 + SGEMM_NOALLOC_PARTIAL_BYTES) + (size_t)first * kSlotTickets;
-    if (!clear) return SGEMM_OK;
-    hipLaunchKernelGGL(clear_tickets, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, s, *tickets, (uint32_t)count);
-    e = hipGetLastError();
-    return e == hipSuccess ? SGEMM_OK : launch_failed(e, "clear_tickets launch");
+    out->partials = reinterpret_cast<float*>(bytes0 + (size_t)out->first * kSlotBytes);
+    out->tickets = reinterpret_cast<uint32_t*>(bytes0 + SGEMM_NOALLOC_PARTIAL_BYTES) + (size_t)out->first * kSlotTickets;
+    if (!fresh && !u.captured) return SGEMM_OK;
+    hipLaunchKernelGGL(clear_tickets, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, s, out->tickets, (uint32_t)count);
+    e = (int)hipGetLastError();
+    return e == 0 ? SGEMM_OK : launch_failed((hipError_t)e, "clear_tickets launch");
 }
 
 }  // namespace
@@ -173,8 +163,7 @@ int sgemm_internal::noalloc_prepare(int dev) {
 void sgemm_internal::noalloc_forget(int dev, hipStream_t stream) {
     if (dev < 0 || dev >= kMaxDevices) return;
     std::lock_guard<std::mutex> lock(g_use_mutex);
-    for (Slot& t : g_use[dev].slots)
-        if (t.owned && t.owner == stream) t.owned = false;
+    (void)g_use[dev].slots.forget(g_use[dev].streams, stream);
 }
 
 extern "C" int sgemm_launch_noalloc(sgemm_handle* h, const float* dA, const float* dB, const float* dC, float* dD,
@@ -190,9 +179,9 @@ extern "C" int sgemm_launch_noalloc(sgemm_handle* h, const float* dA, const floa
                                            n, k, lda, ldb, ldc, ldd, alpha, beta, s);
     sgemm_internal::Part parts[3];
     // the split-BF16 plan never needs more than the scratch
-    const sgemm_internal::SplitPlan sp = sgemm_internal::split_plan(h, m, n, k, lda, ldb, ldc, ldd, alpha, beta);
-    const int count = sp.tile >= 0 ? sgemm_internal::split_strips(h, sp, m, n, lda, ldb, ldc, ldd, parts)
-                                   : sgemm_internal::decompose(h, m, n, k, lda, ldb, ldc, ldd, parts);
+    sgemm_internal::SplitPlan sp = sgemm_internal::split_plan(h, m, n, k, lda, ldb, ldc, ldd, alpha, beta);
+    int count = sp.tile >= 0 ? sgemm_internal::split_strips(h, sp, m, n, lda, ldb, ldc, ldd, parts)
+                             : sgemm_internal::decompose(h, m, n, k, lda, ldb, ldc, ldd, parts);
     // every part's needs are checked before anything is launched
     for (int q = 0; q < count; ++q) {
         const sgemm_internal::Part& pt = parts[q];
@@ -209,13 +198,20 @@ extern "C" int sgemm_launch_noalloc(sgemm_handle* h, const float* dA, const floa
         }
     }
     std::unique_lock<std::mutex> lock(g_use_mutex, std::defer_lock);
+    bool whole = false;   // no scratch for this call: every tile's K in one work-group, by the FP32 kernels
     if (sp.tile >= 0) {
-        float* partials = nullptr;
-        uint32_t* tickets = nullptr;
-        if (sp.partial_bytes && (r = take_scratch(h, sp.partial_bytes, sp.ticket_count, s, lock, &partials, &tickets)) != SGEMM_OK) return r;
-        r = sgemm_internal::bf16x6_launch(sp.tile, sp.splits, sgemm_internal::trans_a(h), sgemm_internal::trans_b(h), dA,
-                                          dB, dC, dD, sp.m, sp.n, k, lda, ldb, ldc, ldd, alpha, beta, partials, tickets, s);
-        if (r != SGEMM_OK) return r;
+        Scratch t;
+        if (sp.partial_bytes && (r = take_scratch(h, sp.partial_bytes, sp.ticket_count, s, lock, &t)) != SGEMM_OK) {
+            if (r != noalloc::kBusy) return r;
+            whole = true;
+            parts[0] = sgemm_internal::Part{h, m, n, 0, 0, 0, 0};
+            count = 1;
+        } else {
+            r = sgemm_internal::bf16x6_launch(sp.tile, sp.splits, sgemm_internal::trans_a(h), sgemm_internal::trans_b(h), dA,
+                                              dB, dC, dD, sp.m, sp.n, k, lda, ldb, ldc, ldd, alpha, beta, t.partials,
+                                              t.tickets, s);
+            if (r != SGEMM_OK) return r;
+        }
     }
     for (int q = 0; q < count; ++q) {
         const sgemm_internal::Part& pt = parts[q];
@@ -224,17 +220,17 @@ extern "C" int sgemm_launch_noalloc(sgemm_handle* h, const float* dA, const floa
         const float* c = dC ? dC + pt.c_off : dC;
         float* d = dD + pt.d_off;
         const sgemm_internal::Plan p = sgemm_internal::plan(pt.kh, pt.m, pt.n, k);
-        if (!p.partial_bytes) {  // generated_gemm uses no workspace
-            r = sgemm_internal::launch(pt.kh, a, b, c, d, pt.m, pt.n, k, lda, ldb, ldc, ldd, alpha, beta, nullptr, s);
-            if (r != SGEMM_OK) return r;
-            continue;
-        }
-        float* partials = nullptr;
-        uint32_t* tickets = nullptr;
         // the parts run in order on one stream, so they share the scratch
-        if ((r = take_scratch(h, p.partial_bytes, p.ticket_count, s, lock, &partials, &tickets)) != SGEMM_OK) return r;
-        const sgemm_internal::Workspace ws{partials, p.partial_bytes, tickets, p.ticket_count};
-        r = sgemm_internal::launch(pt.kh, a, b, c, d, pt.m, pt.n, k, lda, ldb, ldc, ldd, alpha, beta, &ws, s);
+        Scratch t;
+        bool taken = false;
+        if (p.partial_bytes && !whole) {
+            r = take_scratch(h, p.partial_bytes, p.ticket_count, s, lock, &t);
+            if (r != SGEMM_OK && r != noalloc::kBusy) return r;
+            taken = r == SGEMM_OK;
+        }
+        const sgemm_internal::Workspace ws{t.partials, p.partial_bytes, t.tickets, p.ticket_count};
+        r = sgemm_internal::launch(pt.kh, a, b, c, d, pt.m, pt.n, k, lda, ldb, ldc, ldd, alpha, beta, taken ? &ws : nullptr,
+                                   s, !taken);
         if (r != SGEMM_OK) return r;
     }
     return SGEMM_OK;

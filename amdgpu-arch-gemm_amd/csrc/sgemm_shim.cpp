@@ -459,7 +459,7 @@ Plan plan(const sgemm_handle* h, uint32_t m, uint32_t n, uint32_t k) {
 
 int launch(sgemm_handle* h, const float* dA, const float* dB, const float* dC, float* dD, uint32_t m, uint32_t n,
            uint32_t k, uint32_t lda, uint32_t ldb, uint32_t ldc, uint32_t ldd, float alpha, float beta,
-           const Workspace* ws, hipStream_t stream) {
+           const Workspace* ws, hipStream_t stream, bool whole_k) {
     const sgemm_kernel_info& i = h->info;
     KernArgs ka;
     memset(&ka, 0, sizeof(ka));
@@ -469,7 +469,7 @@ int launch(sgemm_handle* h, const float* dA, const float* dB, const float* dC, f
     ka.num_wg_x = (int32_t)((m + (uint32_t)i.tile_m - 1) / (uint32_t)i.tile_m);
     ka.num_wg_y = (int32_t)((n + (uint32_t)i.tile_n - 1) / (uint32_t)i.tile_n);
     const Plan p = plan(h, m, n, k);
-    if (p.splits == 1 && !p.sk_tiles) {
+    if (whole_k || (p.splits == 1 && !p.sk_tiles)) {
         size_t size = sizeof(ka);
         void* extra[] = {HIP_LAUNCH_PARAM_BUFFER_POINTER, &ka, HIP_LAUNCH_PARAM_BUFFER_SIZE, &size, HIP_LAUNCH_PARAM_END};
         HIP_TRY(hipModuleLaunchKernel(h->function, (unsigned)ka.num_wg_x, (unsigned)ka.num_wg_y, 1,

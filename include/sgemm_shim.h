@@ -265,13 +265,14 @@ int sgemm_launch(sgemm_handle* h, const float* dA, const float* dB, const float*
  * (SGEMM_NOALLOC_PARTIAL_BYTES + 4 * SGEMM_NOALLOC_MAX_TILES bytes per device,
  * held until the process ends) instead of the handle's workspace.  A launch
  * needing more partial bytes or tiles than that returns SGEMM_E_SHAPE.  Every
- * call on a device works in that device's array: calls on one stream run one
- * after the other, calls of up to 8 streams side by side when each needs at most
- * an eighth of it, and others wait on the device for those whose part they
- * take over.  Calls
- * under graph capture clear the tickets they use with a kernel of their own
- * (as does every later call on the device); their replays must not overlap
- * other calls on the device or one another. */
+ * eager call on a device works in that device's array: calls on one stream run
+ * one after the other, calls of up to 8 streams side by side when each needs at
+ * most an eighth of it, and others wait on the device for those whose part they
+ * take over.
+ * Calls under graph capture clear the tickets they use with a kernel of their
+ * own (as does every later call on the device); calls on parallel branches
+ * of one captured graph must be ordered by the caller, and replays must not
+ * overlap other calls on the device or one another. */
 int sgemm_launch_noalloc(sgemm_handle* h, const float* dA, const float* dB, const float* dC, float* dD,
                          uint32_t m, uint32_t n, uint32_t k, uint32_t lda, uint32_t ldb, uint32_t ldc, uint32_t ldd,
                          float alpha, float beta);

@@ -1,0 +1,152 @@
+"""sgemm_launch_noalloc between streams that capture: no call spoils another's partial sums.  The rules
+themselves run against a model in test_noalloc_slots.py."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from generator import catalog
+from shim import sgemm_shim as S
+
+pytestmark = pytest.mark.gpu
+
+NAME = "mt64x64_a16_wg1x4_dk32_s3"
+BIG = (640, 640, 8192)       # 100 tiles in 5 K ranges, 8 MB of partials: every slot
+SMALL = (256, 256, 4096)     # 4 MB: one slot
+GLOBAL, THREAD_LOCAL = 0, 1
+_vp = ctypes.c_void_p
+
+
+def _ok(rc):
+    assert rc == 0, rc
+
+
+class _Hip:
+    def __init__(self):
+        self.lib = ctypes.CDLL("libamdhip64.so")
+        for name in ("hipStreamDestroy", "hipStreamSynchronize", "hipGraphExecDestroy", "hipGraphDestroy",
+                     "hipEventDestroy"):
+            getattr(self.lib, name).argtypes = [_vp]
+
+    def stream(self):
+        s = _vp()
+        _ok(self.lib.hipStreamCreate(ctypes.byref(s)))
+        return s
+
+    def begin(self, s, mode=THREAD_LOCAL):
+        _ok(self.lib.hipStreamBeginCapture(s, mode))
+
+    def end(self, s):
+        graph, exe = _vp(), _vp()
+        _ok(self.lib.hipStreamEndCapture(s, ctypes.byref(graph)))
+        _ok(self.lib.hipGraphInstantiate(ctypes.byref(exe), graph, None, None, 0))
+        _ok(self.lib.hipGraphDestroy(graph))
+        return exe
+
+
+class _Call:
+    """One problem's operands, its D and the D that sgemm_launch gives."""
+
+    def __init__(self, shape, seed):
+        m, n, k = self.shape = shape
+        self.a = S.DeviceBuffer.from_array(S.fill_matrix(m, k, seed, 0))
+        self.b = S.DeviceBuffer.from_array(S.fill_matrix(k, n, seed, 1))
+        self.d = S.DeviceBuffer(4 * m * n)
+        with _kernel() as kern:
+            # a slot holds an eighth of the scratch
+            assert (kern.workspace_size(m, n, k) > S.SGEMM_NOALLOC_PARTIAL_BYTES // 8 + 4096) == (shape == BIG)
+            assert kern.launch_splits(m, n, k) > 1
+            kern.launch(self.a, self.b, None, self.d, m, n, k)
+            kern.synchronize()
+        self.want = self.d.download()
+        self.spoil()
+
+    def spoil(self):
+        self.d.upload(np.full(self.want.size, np.nan, dtype=np.float32))
+
+    def run(self, kern):
+        kern.launch_noalloc(self.a, self.b, None, self.d, *self.shape)
+
+    def check(self, what):
+        assert np.array_equal(self.d.download(), self.want), what
+
+
+def _kernel():
+    kern = S.Kernel(*catalog.paths(NAME))
+    kern.set_split_bf16(0)
+    return kern
+
+
+def test_a_captured_call_takes_nothing_over(kernels):
+    hip = _Hip()
+    eager, captured, after = _Call(BIG, 71), _Call(BIG, 72), _Call(BIG, 73)
+    one, two = _kernel(), _kernel()
+    s, t = hip.stream(), hip.stream()
+    exe = _vp()
+    try:
+        one.set_stream(s.value)
+        two.set_stream(t.value)
+        print("capture beside eager calls", flush=True)
+        for r in range(10):
+            eager.run(two)                 # in flight on t ...
+            hip.begin(s)
+            captured.run(one)              # ... while a call that needs every slot is captured on s
+            exe = hip.end(s)
+            after.run(one)                 # and s takes the slots over from t
+            one.synchronize()
+            two.synchronize()
+            eager.check(f"eager {r}")
+            after.check(f"after {r}")
+            for q in range(3):             # the replay, with nothing beside it
+                captured.spoil()
+                _ok(hip.lib.hipGraphLaunch(exe, s))
+                one.synchronize()
+                captured.check(f"replay {r} {q}")
+                after.run(one)
+                one.synchronize()
+                after.check(f"between {r} {q}")
+            _ok(hip.lib.hipGraphExecDestroy(exe))
+            for c in (eager, captured, after):
+                c.spoil()
+    finally:
+        one.close()
+        two.close()
+        hip.lib.hipStreamDestroy(s)
+        hip.lib.hipStreamDestroy(t)
+
+
+def test_split_bf16_calls_share_the_slots(kernels):
+    """K splits of the split-BF16 kernels, small and large, from more streams than slots."""
+    shapes = [(512, 513, 16384), (700, 300, 20000), (1000, 999, 4097)]
+    calls = []
+    for i, (m, n, k) in enumerate(shapes):
+        name = catalog.select(m, n, k)
+        a = S.DeviceBuffer.from_array(S.fill_matrix(m, k, 90 + i, 0))
+        b = S.DeviceBuffer.from_array(S.fill_matrix(k, n, 90 + i, 1))
+        d = S.DeviceBuffer(4 * m * n)
+        with S.Kernel(*catalog.paths(name)) as kern:
+            plan = kern.split_bf16_plan(m, n, k)
+            assert plan and plan["splits"] > 1
+            kern.launch(a, b, None, d, m, n, k)
+            kern.synchronize()
+        calls.append((name, a, b, d.download()))
+    handles = [S.Kernel(*catalog.paths(calls[q % 3][0])) for q in range(10)]
+    try:
+        print("split-BF16 K splits on ten streams", flush=True)
+        for r in range(5):
+            outs = []
+            for q, kern in enumerate(handles):
+                name, a, b, want = calls[q % 3]
+                d = S.DeviceBuffer(want.nbytes)
+                d.upload(np.full(want.size, np.nan, dtype=np.float32))
+                outs.append(d)
+            for q, kern in enumerate(handles):
+                _, a, b, _ = calls[q % 3]
+                kern.launch_noalloc(a, b, None, outs[q], *shapes[q % 3])
+            for kern in handles:
+                kern.synchronize()
+            for q in range(len(handles)):
+                assert np.array_equal(outs[q].download(), calls[q % 3][3]), (r, q)
+    finally:
+        for kern in handles:
+            kern.close()
