@@ -12,8 +12,9 @@
 // graph) and is taken for idle.
 //
 // Captured calls run when their graph is replayed, which is the caller's to
-// order against everything else on the device: they begin at the first slot and
-// leave the owners alone.
+// order against everything else on the device: they leave the owners alone.
+// Those of one capture all begin at the first slot and become a chain of
+// dependent nodes, also where its streams branch.
 #pragma once
 
 #include <cstddef>
@@ -40,7 +41,7 @@ template <class Streams> class Slots {
         uint64_t id = 0;
         *first = 0;
         *fresh = *captured = streams.capturing(s, &id);
-        if (*captured) return 0;
+        if (*captured) return take_captured(streams, s, id);
         auto own = [&](const Slot& t) { return t.state == kOwned && t.owner == s; };
         if (!all)
             for (Slot& t : slots_)
@@ -81,6 +82,8 @@ template <class Streams> class Slots {
 
     // `s`, whose work has ended, is about to be destroyed, or a handle leaves it.
     int forget(Streams&, Stream s) {
+        for (Chain& c : chains_)
+            if (c.last == s) c.on = false;
         for (Slot& t : slots_)
             if (t.state == kOwned && t.owner == s) t.state = kFree;
         return 0;
@@ -93,10 +96,37 @@ template <class Streams> class Slots {
         Stream owner = Stream();
         uint64_t used = 0;
     };
+    // The captured calls of one capture: the stream of the last one.
+    struct Chain {
+        bool on = false;
+        uint64_t id = 0;
+        Stream last = Stream();
+    };
     Slot slots_[kSlots];
     bool was_[kSlots];
     Stream old_[kSlots];
     uint64_t calls_ = 0;
+    Chain chains_[kSlots];   // captures at once; one more runs without scratch
+
+    int take_captured(Streams& streams, Stream s, uint64_t id) {
+        Chain* mine = nullptr;
+        Chain* unused = nullptr;
+        for (Chain& c : chains_) {
+            if (c.on && c.id == id) mine = &c;
+            uint64_t other = 0;
+            if (!c.on || (c.id != id && !(streams.capturing(c.last, &other) && other == c.id))) unused = &c;
+        }
+        if (mine && !(mine->last == s)) {
+            const int e = streams.order(mine->last, s);
+            if (e) return e;
+        }
+        if (!mine) mine = unused;
+        if (!mine) return kBusy;
+        mine->on = true;
+        mine->id = id;
+        mine->last = s;
+        return 0;
+    }
 };
 
 }  // namespace noalloc

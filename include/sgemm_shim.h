@@ -270,8 +270,8 @@ int sgemm_launch(sgemm_handle* h, const float* dA, const float* dB, const float*
  * most an eighth of it, and others wait on the device for those whose part they
  * take over.
  * Calls under graph capture clear the tickets they use with a kernel of their
- * own (as does every later call on the device); calls on parallel branches
- * of one captured graph must be ordered by the caller, and replays must not
+ * own (as does every later call on the device); calls of one capture
+ * become dependent nodes, on parallel branches too.  Their replays must not
  * overlap other calls on the device or one another. */
 int sgemm_launch_noalloc(sgemm_handle* h, const float* dA, const float* dB, const float* dC, float* dD,
                          uint32_t m, uint32_t n, uint32_t k, uint32_t lda, uint32_t ldb, uint32_t ldc, uint32_t ldd,

@@ -1,4 +1,4 @@
-"""sgemm_launch_noalloc between streams that capture: no call spoils another's partial sums.  The rules
+"""sgemm_launch_noalloc between streams that capture and fork: no call spoils another's partial sums.  The rules
 themselves run against a model in test_noalloc_slots.py."""
 import ctypes
 
@@ -32,6 +32,11 @@ class _Hip:
         s = _vp()
         _ok(self.lib.hipStreamCreate(ctypes.byref(s)))
         return s
+
+    def event(self):
+        e = _vp()
+        _ok(self.lib.hipEventCreateWithFlags(ctypes.byref(e), 2))
+        return e
 
     def begin(self, s, mode=THREAD_LOCAL):
         _ok(self.lib.hipStreamBeginCapture(s, mode))
@@ -111,6 +116,44 @@ def test_a_captured_call_takes_nothing_over(kernels):
     finally:
         one.close()
         two.close()
+        hip.lib.hipStreamDestroy(s)
+        hip.lib.hipStreamDestroy(t)
+
+
+def test_branches_of_one_capture_are_a_chain(kernels):
+    hip = _Hip()
+    calls = [_Call(BIG, 74), _Call(BIG, 75), _Call(SMALL, 76), _Call(SMALL, 77)]
+    one, two = _kernel(), _kernel()
+    s, t = hip.stream(), hip.stream()
+    fork, join = hip.event(), hip.event()
+    exe = _vp()
+    try:
+        one.set_stream(s.value)
+        two.set_stream(t.value)
+        print("two branches in one capture", flush=True)
+        hip.begin(s)
+        _ok(hip.lib.hipEventRecord(fork, s))
+        _ok(hip.lib.hipStreamWaitEvent(t, fork, 0))
+        for i, c in enumerate(calls):      # the branches take turns, no edge between them from here
+            c.run((one, two)[i % 2])
+        _ok(hip.lib.hipEventRecord(join, t))
+        _ok(hip.lib.hipStreamWaitEvent(s, join, 0))
+        exe = hip.end(s)
+        for q in range(5):
+            for c in calls:
+                c.spoil()
+            _ok(hip.lib.hipGraphLaunch(exe, s))
+            one.synchronize()
+            for i, c in enumerate(calls):
+                c.check(f"replay {q} call {i}")
+            calls[2].run(two)              # eager work between the replays
+            two.synchronize()
+        _ok(hip.lib.hipGraphExecDestroy(exe))
+    finally:
+        one.close()
+        two.close()
+        for e in (fork, join):
+            hip.lib.hipEventDestroy(e)
         hip.lib.hipStreamDestroy(s)
         hip.lib.hipStreamDestroy(t)
 

@@ -167,6 +167,7 @@ def model(tmp_path_factory):
 @pytest.mark.parametrize("events", [
     [],
     ["captures"],                                     # a captured call leaves the eager owners alone
+    ["captures", "forks"],                            # two branches of one capture meet in a slot
 ])
 def test_launches_that_share_a_slot_are_ordered(model, events):
     ret = subprocess.run([model] + events, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, timeout=120)
