@@ -8,8 +8,10 @@
 // owner is waited for on the device, by an event recorded on its stream when the
 // slot is taken over: a call on a slot that its stream owns costs nothing.
 //
-// A stream that is capturing cannot be recorded on (the event would join its
-// graph) and is taken for idle.
+// A stream that is capturing can neither be recorded on (the event would join
+// its graph) nor be assumed idle (eager calls from before its capture may still
+// run), so its slots cannot be taken over: a call that needs one gets kBusy and
+// runs without scratch.
 //
 // Captured calls run when their graph is replayed, which is the caller's to
 // order against everything else on the device: they leave the owners alone.
@@ -28,7 +30,8 @@ constexpr int kBusy = -1000;   // no scratch for this call now
 // Streams:
 //   typedef ... Stream;
 //   bool capturing(Stream s, uint64_t* id)   whether s is capturing, in which capture
-//   int order(Stream before, Stream after)   later work of `after` waits for the work enqueued on `before`
+//   int order(Stream before, Stream after)   later work of `after` waits for the work enqueued on `before`;
+//                                            kBusy: `before` began a capture meanwhile, nothing waits
 // and every int is 0 on success.
 template <class Streams> class Slots {
   public:
@@ -51,17 +54,22 @@ template <class Streams> class Slots {
                     return 0;
                 }
         uint64_t other = 0;
+        bool stuck[kSlots];
+        for (int q = 0; q < kSlots; ++q)
+            stuck[q] = slots_[q].state == kOwned && !own(slots_[q]) && streams.capturing(slots_[q].owner, &other);
         if (!all) {
-            auto rank = [&](int q) { return slots_[q].state == kFree ? 1 : 2; };
+            auto rank = [&](int q) { return slots_[q].state == kFree ? 1 : !stuck[q] ? 2 : 3; };
             for (int q = 1; q < kSlots; ++q)
                 if (rank(q) < rank(*first) || (rank(q) == rank(*first) && slots_[q].used < slots_[*first].used)) *first = q;
         }
         const int end = all ? kSlots : *first + 1;
+        for (int q = *first; q < end; ++q)
+            if (stuck[q]) return kBusy;
         for (int q = *first; q < end; ++q) {
             Slot& t = slots_[q];
             if (!own(t)) {
                 *fresh = true;
-                bool waited = t.state == kFree || streams.capturing(t.owner, &other);
+                bool waited = t.state == kFree;
                 for (int p = *first; p < q && !waited; ++p) waited = t.state == kOwned && was_[p] && old_[p] == t.owner;
                 if (!waited) {
                     const int e = streams.order(t.owner, s);

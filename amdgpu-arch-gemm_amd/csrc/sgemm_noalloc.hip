@@ -74,6 +74,8 @@ struct HipStreams {
     int order(hipStream_t before, hipStream_t after) {
         hipError_t e = hipEventRecord(moment, before);
         if (e != hipSuccess) return (int)e;
+        uint64_t x = 0, y = 0;
+        if (capturing(before, &x) && !(capturing(after, &y) && x == y)) return noalloc::kBusy;
         return (int)hipStreamWaitEvent(after, moment, 0);
     }
     hipError_t create() {

@@ -269,6 +269,9 @@ int sgemm_launch(sgemm_handle* h, const float* dA, const float* dB, const float*
  * one after the other, calls of up to 8 streams side by side when each needs at
  * most an eighth of it, and others wait on the device for those whose part they
  * take over.
+ * While a stream captures, its eager calls from before cannot be waited
+ * for: a call that needs their part then runs without scratch, each tile's K in
+ * one work-group (right, but slower and not the bits of sgemm_launch).
  * Calls under graph capture clear the tickets they use with a kernel of their
  * own (as does every later call on the device); calls of one capture
  * become dependent nodes, on parallel branches too.  Their replays must not

@@ -158,6 +158,53 @@ def test_branches_of_one_capture_are_a_chain(kernels):
         hip.lib.hipStreamDestroy(t)
 
 
+def test_a_capturing_owner_keeps_its_slots(kernels):
+    """The owner's eager call may still run while it captures: a call that needs
+    its slots runs without scratch, each tile's K in one work-group."""
+    hip = _Hip()
+    first, captured, other, small = _Call(BIG, 78), _Call(BIG, 79), _Call(BIG, 80), _Call(SMALL, 81)
+    one, two = _kernel(), _kernel()
+    s = hip.stream()
+    try:
+        two.set_stream(s.value)
+        whole = []
+        one.set_split_k(1)
+        for c in (other, small):
+            one.launch(c.a, c.b, None, c.d, *c.shape)
+            one.synchronize()
+            whole.append(c.d.download())
+            assert not np.array_equal(whole[-1], c.want)
+        one.set_split_k(0)
+        print("an owner that captures", flush=True)
+        for r in range(5):
+            first.run(two)
+            hip.begin(s)
+            captured.run(two)
+            other.run(one)                 # every slot is the capturing stream's
+            small.run(one)
+            exe = hip.end(s)
+            one.synchronize()
+            two.synchronize()
+            first.check(f"first {r}")
+            for c, w in zip((other, small), whole):
+                assert np.array_equal(c.d.download(), w), r
+            for q in range(3):
+                captured.spoil()
+                _ok(hip.lib.hipGraphLaunch(exe, s))
+                two.synchronize()
+                captured.check(f"replay {r} {q}")
+            _ok(hip.lib.hipGraphExecDestroy(exe))
+            other.run(one)                 # the capture has ended: with scratch again
+            one.synchronize()
+            other.check(f"other {r}")
+            first.run(two)                 # and the slots are the first stream's again
+            two.synchronize()
+    finally:
+        one.close()
+        two.close()
+        hip.lib.hipStreamDestroy(s)
+
+
 def test_split_bf16_calls_share_the_slots(kernels):
     """K splits of the split-BF16 kernels, small and large, from more streams than slots."""
     shapes = [(512, 513, 16384), (700, 300, 20000), (1000, 999, 4097)]
