@@ -32,6 +32,7 @@ constexpr int kBusy = -1000;   // no scratch for this call now
 //   bool capturing(Stream s, uint64_t* id)   whether s is capturing, in which capture
 //   int order(Stream before, Stream after)   later work of `after` waits for the work enqueued on `before`;
 //                                            kBusy: `before` began a capture meanwhile, nothing waits
+//   int sync(Stream s)                       waits for s on the host
 // and every int is 0 on success.
 template <class Streams> class Slots {
   public:
@@ -88,13 +89,19 @@ template <class Streams> class Slots {
         return 0;
     }
 
-    // `s`, whose work has ended, is about to be destroyed, or a handle leaves it.
-    int forget(Streams&, Stream s) {
+    // `s` is about to be destroyed, or a handle leaves it: its slots are free
+    // once its work has ended (calls of other handles on it included, which the
+    // lock keeps out meanwhile).
+    int forget(Streams& streams, Stream s) {
+        bool any = false;
+        for (const Slot& t : slots_) any = any || (t.state == kOwned && t.owner == s);
         for (Chain& c : chains_)
             if (c.last == s) c.on = false;
+        if (!any) return 0;
+        const int e = streams.sync(s);
         for (Slot& t : slots_)
             if (t.state == kOwned && t.owner == s) t.state = kFree;
-        return 0;
+        return e;
     }
 
   private:

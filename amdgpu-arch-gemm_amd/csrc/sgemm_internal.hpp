@@ -108,7 +108,8 @@ SGEMM_INTERNAL __attribute__((weak)) int thin_prepare();   // the same for the t
 // calls it for the handle's device, so launches never do.
 SGEMM_INTERNAL int noalloc_prepare(int dev);
 // A stream that is about to be destroyed (or that a handle leaves) orders no
-// later call: another stream may get its address.  Weak, as bf16x6_launch.
+// later call: another stream may get its address.  Waits for the stream if it
+// owns some of the scratch.  Weak, as bf16x6_launch.
 SGEMM_INTERNAL __attribute__((weak)) void noalloc_forget(int dev, hipStream_t stream);
 
 SGEMM_INTERNAL hipStream_t stream(const sgemm_handle* h);

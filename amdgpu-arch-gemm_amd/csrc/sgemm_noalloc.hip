@@ -78,6 +78,7 @@ struct HipStreams {
         if (capturing(before, &x) && !(capturing(after, &y) && x == y)) return noalloc::kBusy;
         return (int)hipStreamWaitEvent(after, moment, 0);
     }
+    int sync(hipStream_t s) { return (int)hipStreamSynchronize(s); }
     hipError_t create() {
         return moment ? hipSuccess : hipEventCreateWithFlags(&moment, hipEventDisableTiming);
     }

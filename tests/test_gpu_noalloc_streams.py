@@ -1,6 +1,7 @@
-"""sgemm_launch_noalloc between streams that capture and fork: no call spoils another's partial sums.  The rules
+"""sgemm_launch_noalloc between streams that capture, fork or are shared: no call spoils another's partial sums.  The rules
 themselves run against a model in test_noalloc_slots.py."""
 import ctypes
+import threading
 
 import numpy as np
 import pytest
@@ -202,6 +203,35 @@ def test_a_capturing_owner_keeps_its_slots(kernels):
     finally:
         one.close()
         two.close()
+        hip.lib.hipStreamDestroy(s)
+
+
+def test_a_handle_leaves_a_stream_that_others_use(kernels):
+    hip = _Hip()
+    a, b, c = _Call(BIG, 82), _Call(SMALL, 83), _Call(BIG, 84)
+    s = hip.stream()
+    two, three = _kernel(), _kernel()
+    try:
+        two.set_stream(s.value)
+        print("a shared stream", flush=True)
+        for r in range(10):
+            one = _kernel()
+            one.set_stream(s.value)
+            b.run(one)
+            leaver = threading.Thread(target=one.close)   # while `two` keeps launching on the stream
+            leaver.start()
+            a.run(two)
+            c.run(three)                   # from a third stream, over a's slots
+            leaver.join()
+            c.run(three)
+            two.synchronize()
+            three.synchronize()
+            for i, x in enumerate((a, b, c)):
+                x.check(f"{r} {i}")
+                x.spoil()
+    finally:
+        two.close()
+        three.close()
         hip.lib.hipStreamDestroy(s)
 
 

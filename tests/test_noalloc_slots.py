@@ -170,7 +170,8 @@ def model(tmp_path_factory):
     ["captures", "forks"],                            # two branches of one capture meet in a slot
     ["captures", "eager_before"],                     # an owner captures while its eager calls still run
     ["captures", "captures_race"],                    # ... or begins to while it is recorded on
-    ["captures", "forks", "eager_before", "captures_race"],
+    ["leaves"],                                       # a stream shared by two handles, one of which leaves it
+    ["captures", "forks", "eager_before", "captures_race", "leaves"],
 ])
 def test_launches_that_share_a_slot_are_ordered(model, events):
     ret = subprocess.run([model] + events, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, timeout=120)
