@@ -17,6 +17,10 @@
 // order against everything else on the device: they leave the owners alone.
 // Those of one capture all begin at the first slot and become a chain of
 // dependent nodes, also where its streams branch.
+//
+// A name that stands for another stream in every thread (hipStreamPerThread)
+// cannot be recorded on later from elsewhere: its calls record the slot's own
+// event at once, which every later call on the slot waits for.
 #pragma once
 
 #include <cstddef>
@@ -30,8 +34,12 @@ constexpr int kBusy = -1000;   // no scratch for this call now
 // Streams:
 //   typedef ... Stream;
 //   bool capturing(Stream s, uint64_t* id)   whether s is capturing, in which capture
+//   bool per_thread(Stream s)                whether the name means another stream in every thread
+//   uint64_t thread()                        the calling thread
 //   int order(Stream before, Stream after)   later work of `after` waits for the work enqueued on `before`;
 //                                            kBusy: `before` began a capture meanwhile, nothing waits
+//   int mark(int slot, Stream s)             the slot's event: the work enqueued on s so far
+//   int wait(int slot, Stream s)             later work of s waits for the slot's event
 //   int sync(Stream s)                       waits for s on the host
 // and every int is 0 on success.
 template <class Streams> class Slots {
@@ -46,7 +54,8 @@ template <class Streams> class Slots {
         *first = 0;
         *fresh = *captured = streams.capturing(s, &id);
         if (*captured) return take_captured(streams, s, id);
-        auto own = [&](const Slot& t) { return t.state == kOwned && t.owner == s; };
+        const bool named = streams.per_thread(s);
+        auto own = [&](const Slot& t) { return t.state == kOwned && t.owner == s && !named; };
         if (!all)
             for (Slot& t : slots_)
                 if (own(t)) {
@@ -73,7 +82,7 @@ template <class Streams> class Slots {
                 bool waited = t.state == kFree;
                 for (int p = *first; p < q && !waited; ++p) waited = t.state == kOwned && was_[p] && old_[p] == t.owner;
                 if (!waited) {
-                    const int e = streams.order(t.owner, s);
+                    const int e = t.state == kMarked ? streams.wait(q, s) : streams.order(t.owner, s);
                     if (e) return e;
                 }
             }
@@ -86,6 +95,18 @@ template <class Streams> class Slots {
             slots_[q].used = calls_ + 1;
         }
         ++calls_;
+        return 0;
+    }
+
+    // After the call's launch on `s` (same lock as its take).
+    int done(Streams& streams, Stream s, bool all, int first) {
+        uint64_t id = 0;
+        if (!streams.per_thread(s) || streams.capturing(s, &id)) return 0;
+        for (int q = first; q < (all ? kSlots : first + 1); ++q) {
+            const int e = streams.mark(q, s);
+            if (e) return e;
+            slots_[q].state = kMarked;
+        }
         return 0;
     }
 
@@ -105,16 +126,17 @@ template <class Streams> class Slots {
     }
 
   private:
-    enum State { kFree, kOwned };
+    enum State { kFree, kOwned, kMarked };
     struct Slot {
         State state = kFree;
         Stream owner = Stream();
         uint64_t used = 0;
     };
-    // The captured calls of one capture: the stream of the last one.
+    // The captured calls of one capture: the stream (and thread, for a
+    // per-thread name) of the last one.
     struct Chain {
         bool on = false;
-        uint64_t id = 0;
+        uint64_t id = 0, thread = 0;
         Stream last = Stream();
     };
     Slot slots_[kSlots];
@@ -124,14 +146,17 @@ template <class Streams> class Slots {
     Chain chains_[kSlots];   // captures at once; one more runs without scratch
 
     int take_captured(Streams& streams, Stream s, uint64_t id) {
+        const uint64_t thread = streams.per_thread(s) ? streams.thread() : 0;
         Chain* mine = nullptr;
         Chain* unused = nullptr;
         for (Chain& c : chains_) {
             if (c.on && c.id == id) mine = &c;
             uint64_t other = 0;
-            if (!c.on || (c.id != id && !(streams.capturing(c.last, &other) && other == c.id))) unused = &c;
+            const bool elsewhere = c.thread && c.thread != streams.thread();   // cannot be asked from here
+            if (!c.on || (!elsewhere && c.id != id && !(streams.capturing(c.last, &other) && other == c.id))) unused = &c;
         }
-        if (mine && !(mine->last == s)) {
+        if (mine && !(mine->last == s && mine->thread == thread)) {
+            if (mine->thread && mine->thread != streams.thread()) return kBusy;
             const int e = streams.order(mine->last, s);
             if (e) return e;
         }
@@ -140,6 +165,7 @@ template <class Streams> class Slots {
         mine->on = true;
         mine->id = id;
         mine->last = s;
+        mine->thread = thread;
         return 0;
     }
 };

@@ -21,7 +21,9 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdio>
+#include <functional>
 #include <mutex>
+#include <thread>
 
 static_assert(bf16x6::kMaxPartialBytes <= SGEMM_NOALLOC_PARTIAL_BYTES && bf16x6::kMaxTickets <= SGEMM_NOALLOC_MAX_TILES,
               "every split-BF16 plan fits the static scratch");
@@ -62,6 +64,7 @@ constexpr size_t kSlotTickets = (size_t)SGEMM_NOALLOC_MAX_TILES / noalloc::kSlot
 struct HipStreams {
     typedef hipStream_t Stream;
     hipEvent_t moment = nullptr;                 // recorded and waited for within one order()
+    hipEvent_t marks[noalloc::kSlots] = {};
 
     bool capturing(hipStream_t s, uint64_t* id) {
         hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
@@ -71,6 +74,8 @@ struct HipStreams {
         *id = n;
         return on;
     }
+    bool per_thread(hipStream_t s) { return s == hipStreamPerThread; }
+    uint64_t thread() { return std::hash<std::thread::id>()(std::this_thread::get_id()) | 1u; }
     int order(hipStream_t before, hipStream_t after) {
         hipError_t e = hipEventRecord(moment, before);
         if (e != hipSuccess) return (int)e;
@@ -78,9 +83,14 @@ struct HipStreams {
         if (capturing(before, &x) && !(capturing(after, &y) && x == y)) return noalloc::kBusy;
         return (int)hipStreamWaitEvent(after, moment, 0);
     }
+    int mark(int slot, hipStream_t s) { return (int)hipEventRecord(marks[slot], s); }
+    int wait(int slot, hipStream_t s) { return (int)hipStreamWaitEvent(s, marks[slot], 0); }
     int sync(hipStream_t s) { return (int)hipStreamSynchronize(s); }
     hipError_t create() {
-        return moment ? hipSuccess : hipEventCreateWithFlags(&moment, hipEventDisableTiming);
+        hipError_t e = moment ? hipSuccess : hipEventCreateWithFlags(&moment, hipEventDisableTiming);
+        for (hipEvent_t& m : marks)
+            if (e == hipSuccess && !m) e = hipEventCreateWithFlags(&m, hipEventDisableTiming);
+        return e;
     }
 };
 
@@ -132,7 +142,8 @@ struct Scratch {
 };
 
 // Partials (`bytes`) and tickets (`count`, zero) on h's device for the launch
-// that the caller enqueues on `s` next, with `lock` still held.  noalloc::kBusy: none now.
+// that the caller enqueues on `s` next, with `lock` still held, before it calls
+// give_scratch.  noalloc::kBusy: none now.
 int take_scratch(const sgemm_handle* h, size_t bytes, size_t count, hipStream_t s, std::unique_lock<std::mutex>& lock,
                  Scratch* out) {
     const int dev = sgemm_internal::device(h);
@@ -154,6 +165,13 @@ int take_scratch(const sgemm_handle* h, size_t bytes, size_t count, hipStream_t 
     hipLaunchKernelGGL(clear_tickets, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, s, out->tickets, (uint32_t)count);
     e = (int)hipGetLastError();
     return e == 0 ? SGEMM_OK : launch_failed((hipError_t)e, "clear_tickets launch");
+}
+
+// After the launch that take_scratch was called for (its result `r`).
+int give_scratch(const sgemm_handle* h, hipStream_t s, const Scratch& t, int r) {
+    Use& u = g_use[sgemm_internal::device(h)];
+    const int e = u.slots.done(u.streams, s, t.all, t.first);
+    return r != SGEMM_OK || !e ? r : launch_failed((hipError_t)e, "ordering two streams' calls");
 }
 
 }  // namespace
@@ -213,6 +231,7 @@ extern "C" int sgemm_launch_noalloc(sgemm_handle* h, const float* dA, const floa
             r = sgemm_internal::bf16x6_launch(sp.tile, sp.splits, sgemm_internal::trans_a(h), sgemm_internal::trans_b(h), dA,
                                               dB, dC, dD, sp.m, sp.n, k, lda, ldb, ldc, ldd, alpha, beta, t.partials,
                                               t.tickets, s);
+            if (sp.partial_bytes) r = give_scratch(h, s, t, r);
             if (r != SGEMM_OK) return r;
         }
     }
@@ -234,6 +253,7 @@ extern "C" int sgemm_launch_noalloc(sgemm_handle* h, const float* dA, const floa
         const sgemm_internal::Workspace ws{t.partials, p.partial_bytes, t.tickets, p.ticket_count};
         r = sgemm_internal::launch(pt.kh, a, b, c, d, pt.m, pt.n, k, lda, ldb, ldc, ldd, alpha, beta, taken ? &ws : nullptr,
                                    s, !taken);
+        if (taken) r = give_scratch(h, s, t, r);
         if (r != SGEMM_OK) return r;
     }
     return SGEMM_OK;

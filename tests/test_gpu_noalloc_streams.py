@@ -1,4 +1,5 @@
-"""sgemm_launch_noalloc between streams that capture, fork or are shared: no call spoils another's partial sums.  The rules
+"""sgemm_launch_noalloc between streams that capture, fork, are shared or stand
+for one stream per thread: no call spoils another's partial sums.  The rules
 themselves run against a model in test_noalloc_slots.py."""
 import ctypes
 import threading
@@ -15,6 +16,7 @@ NAME = "mt64x64_a16_wg1x4_dk32_s3"
 BIG = (640, 640, 8192)       # 100 tiles in 5 K ranges, 8 MB of partials: every slot
 SMALL = (256, 256, 4096)     # 4 MB: one slot
 GLOBAL, THREAD_LOCAL = 0, 1
+PER_THREAD = 2               # hipStreamPerThread
 _vp = ctypes.c_void_p
 
 
@@ -233,6 +235,37 @@ def test_a_handle_leaves_a_stream_that_others_use(kernels):
         two.close()
         three.close()
         hip.lib.hipStreamDestroy(s)
+
+
+def test_one_name_for_a_stream_of_every_thread(kernels):
+    calls = [[_Call(SMALL, 85), _Call(BIG, 86)], [_Call(SMALL, 87), _Call(BIG, 88)]]
+    handles = [_kernel(), _kernel()]
+    failed = []
+
+    def work(q):
+        try:
+            handles[q].set_stream(PER_THREAD)
+            for _ in range(20):
+                for c in calls[q]:
+                    c.run(handles[q])
+            handles[q].synchronize()
+            for i, c in enumerate(calls[q]):
+                c.check(f"thread {q} call {i}")
+            handles[q].set_stream(None)
+        except BaseException as e:   # reported by the test's own thread
+            failed.append(e)
+
+    print("two threads on their own per-thread streams", flush=True)
+    threads = [threading.Thread(target=work, args=(q,)) for q in range(2)]
+    try:
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        assert not failed, failed
+    finally:
+        for h in handles:
+            h.close()
 
 
 def test_split_bf16_calls_share_the_slots(kernels):

@@ -96,6 +96,7 @@ int main(int argc, char** argv) {
             }
             if (e) m.die("error");
             m.launch(s, first, all ? kSlots : first + 1);
+            slots.done(m, s, all, first);
         };
         const int streams = 2 + (int)(rng() % 11);
         for (int step = 0; step < 120; ++step) {
@@ -171,7 +172,8 @@ def model(tmp_path_factory):
     ["captures", "eager_before"],                     # an owner captures while its eager calls still run
     ["captures", "captures_race"],                    # ... or begins to while it is recorded on
     ["leaves"],                                       # a stream shared by two handles, one of which leaves it
-    ["captures", "forks", "eager_before", "captures_race", "leaves"],
+    ["per_thread"],                                   # one name, a stream in every thread
+    ["captures", "forks", "eager_before", "captures_race", "leaves", "per_thread"],
 ])
 def test_launches_that_share_a_slot_are_ordered(model, events):
     ret = subprocess.run([model] + events, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, timeout=120)
