@@ -984,6 +984,11 @@ int grow_workspace(sgemm_handle* kh, hipStream_t stream, size_t ws_need, size_t 
     return SGEMM_OK;
 }
 
+bool is_capturing(hipStream_t stream) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone;
+}
+
 // One part of a launch on `stream` with kernel handle `kh`.
 int launch_part(sgemm_handle* kh, hipStream_t stream, const float* dA, const float* dB, const float* dC, float* dD,
                 uint32_t m, uint32_t n, uint32_t k, uint32_t lda, uint32_t ldb, uint32_t ldc, uint32_t ldd, float alpha,
@@ -1010,7 +1015,13 @@ int sgemm_launch(sgemm_handle* h, const float* dA, const float* dB, const float*
         return sgemm_internal::thin_launch(ts, h->info.trans_a != 0, h->info.trans_b != 0, dA, dB, dC, dD, m, n, k, lda,
                                            ldb, ldc, ldd, alpha, beta, h->stream);
     sgemm_internal::Part parts[3];
-    const sgemm_internal::SplitPlan sp = sgemm_internal::split_plan(h, m, n, k, lda, ldb, ldc, ldd, alpha, beta);
+    sgemm_internal::SplitPlan sp = sgemm_internal::split_plan(h, m, n, k, lda, ldb, ldc, ldd, alpha, beta);
+    // A plan whose workspace cannot be had (under capture, which no allocation
+    // may join, or for want of memory) leaves the call to h's own kernels, which
+    // may need none.
+    if (sp.tile >= 0 && (h->ws_bytes < sp.partial_bytes || h->ticket_count < sp.ticket_count) &&
+        (is_capturing(h->stream) || grow_workspace(h, h->stream, sp.partial_bytes, sp.ticket_count) != SGEMM_OK))
+        sp = sgemm_internal::SplitPlan();
     int count = sp.tile >= 0 ? sgemm_internal::split_strips(h, sp, m, n, lda, ldb, ldc, ldd, parts)
                              : sgemm_internal::decompose(h, m, n, k, lda, ldb, ldc, ldd, parts);
     for (int q = 0; q < count; ++q) {
@@ -1018,7 +1029,6 @@ int sgemm_launch(sgemm_handle* h, const float* dA, const float* dB, const float*
         if (pt.kh != h && (r = sgemm_check_shape(pt.kh, pt.m, pt.n, k, lda, ldb, ldc, ldd)) != SGEMM_OK) return r;
     }
     if (sp.tile >= 0) {
-        if ((r = grow_workspace(h, h->stream, sp.partial_bytes, sp.ticket_count)) != SGEMM_OK) return r;
         r = sgemm_internal::bf16x6_launch(sp.tile, sp.splits, h->info.trans_a != 0, h->info.trans_b != 0, dA, dB, dC, dD,
                                           sp.m, sp.n, k, lda, ldb, ldc, ldd, alpha, beta, (float*)h->ws, h->tickets,
                                           h->stream);
