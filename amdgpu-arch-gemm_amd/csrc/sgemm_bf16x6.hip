@@ -52,12 +52,13 @@ bool g_loaded[kMaxDevices];  // devices that hold the kernels
 
 template <template <bool, bool> class T>
 hipError_t launch_tile(bool ta, bool tb, const Args& p, hipStream_t stream) {
+    // The launch's own result, not hipGetLastError: that may still hold an error
+    // of an earlier call of the program.
     const dim3 grid((unsigned)p.nwgx * (unsigned)p.nwgy, p.splits), block(T<false, false>::NT);
-    if (ta && tb) hipLaunchKernelGGL((bf16x6::kernel<T<true, true>>), grid, block, 0, stream, p);
-    else if (ta) hipLaunchKernelGGL((bf16x6::kernel<T<true, false>>), grid, block, 0, stream, p);
-    else if (tb) hipLaunchKernelGGL((bf16x6::kernel<T<false, true>>), grid, block, 0, stream, p);
-    else hipLaunchKernelGGL((bf16x6::kernel<T<false, false>>), grid, block, 0, stream, p);
-    return hipGetLastError();
+    void (*const f)(Args) = ta ? (tb ? bf16x6::kernel<T<true, true>> : bf16x6::kernel<T<true, false>>)
+                               : (tb ? bf16x6::kernel<T<false, true>> : bf16x6::kernel<T<false, false>>);
+    void* args[] = {const_cast<Args*>(&p)};
+    return hipLaunchKernel(reinterpret_cast<const void*>(f), grid, block, args, 0, stream);
 }
 
 }  // namespace

@@ -162,8 +162,9 @@ int take_scratch(const sgemm_handle* h, size_t bytes, size_t count, hipStream_t 
     out->partials = reinterpret_cast<float*>(bytes0 + (size_t)out->first * kSlotBytes);
     out->tickets = reinterpret_cast<uint32_t*>(bytes0 + SGEMM_NOALLOC_PARTIAL_BYTES) + (size_t)out->first * kSlotTickets;
     if (!fresh && !u.captured) return SGEMM_OK;
-    hipLaunchKernelGGL(clear_tickets, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, s, out->tickets, (uint32_t)count);
-    e = (int)hipGetLastError();
+    uint32_t n = (uint32_t)count;
+    void* args[] = {&out->tickets, &n};
+    e = (int)hipLaunchKernel(reinterpret_cast<const void*>(&clear_tickets), dim3((n + 255) / 256), dim3(256), args, 0, s);
     return e == 0 ? SGEMM_OK : launch_failed((hipError_t)e, "clear_tickets launch");
 }
 

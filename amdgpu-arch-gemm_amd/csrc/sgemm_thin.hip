@@ -223,8 +223,10 @@ __global__ void __launch_bounds__(1024) thin_kernel(const Args p) {
 
 template <int XA, bool XKC, bool YKC, bool X_IS_A> hipError_t go(const Args& p, int waves, hipStream_t s) {
     const size_t lds = (size_t)waves * XA * 1024;
-    hipLaunchKernelGGL((thin_kernel<XA, XKC, YKC, X_IS_A>), dim3((p.rows + 16 * XA - 1) / (16 * XA)), dim3(64 * waves), lds, s, p);
-    return hipGetLastError();
+    // its own result: hipGetLastError may still hold an earlier call's error
+    void* args[] = {const_cast<Args*>(&p)};
+    return hipLaunchKernel(reinterpret_cast<const void*>(&thin_kernel<XA, XKC, YKC, X_IS_A>),
+                           dim3((p.rows + 16 * XA - 1) / (16 * XA)), dim3(64 * waves), args, lds, s);
 }
 
 template <bool XKC, bool YKC, bool X_IS_A> hipError_t pick(const Args& p, const thin::Shape& t, hipStream_t s) {

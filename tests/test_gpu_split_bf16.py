@@ -1,5 +1,7 @@
 """The split-BF16 kernels (csrc/bf16x6_kernel.hpp) through the public launch
 path, against float64 and against the same handle's FP32 kernels."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -171,3 +173,30 @@ def test_split_bf16_is_off_where_the_handle_is_fixed(kernels):
             e.close()
     with S.Kernel(*catalog.paths("mt256x256_a32_wg2x2_dk16")) as other:      # no split_bf16 key
         assert other.split_bf16_plan(m, n, k) is None
+
+
+@pytest.mark.parametrize("m,n,k,entry", [(2048, 2048, 512, "launch"), (1000, 999, 4097, "launch_noalloc"),
+                                         (2048, 8, 1024, "launch"), (333, 129, 517, "launch_noalloc")])
+def test_an_earlier_error_is_not_the_launchs(kernels, m, n, k, entry):
+    """The split, thin and ticket-clearing kernels report their own launch: an
+    error that the program left behind before (here a device that does not
+    exist) must not fail them."""
+    print(f"stale error {m}x{n}x{k} {entry}", flush=True)
+    hip = ctypes.CDLL("libamdhip64.so")
+    a, b = (S.DeviceBuffer.from_array(S.fill_matrix(*s, 56, i)) for i, s in enumerate(((m, k), (k, n))))
+    d = S.DeviceBuffer(4 * m * n)
+    kern, edges = _handles(m, n, k, "nn")
+    try:
+        kern.launch(a, b, None, d, m, n, k)
+        kern.synchronize()
+        want = d.download()
+        d.upload(np.full(m * n, np.nan, dtype=np.float32))
+        assert hip.hipSetDevice(9999) != 0
+        getattr(kern, entry)(a, b, None, d, m, n, k)
+        hip.hipGetLastError()
+        kern.synchronize()
+        assert np.array_equal(d.download(), want)
+    finally:
+        kern.close()
+        for e in edges:
+            e.close()
