@@ -606,7 +606,14 @@ SplitPlan split_plan(const sgemm_handle* h, uint32_t m, uint32_t n, uint32_t k, 
     // kernels: one row or column more would be a tile row or column more
     const uint32_t me = h->edge_rows && m > 128 && m % 128 && m % 128 <= 16 ? m % 128 : 0u;
     const uint32_t ne = h->edge_cols && n > 128 && n % 128 && n % 128 <= 16 ? n % 128 : 0u;
-    if (me || ne)
+    // (an edge kernel may refuse what h's own accepts: a grid of its narrower tiles can be too large)
+    auto accepts = [&](const sgemm_handle* e, uint32_t pm, uint32_t pn) {
+        const std::string last = g_last_error;
+        const bool yes = sgemm_check_shape(e, pm, pn, k, lda, ldb, ldc, ldd) == SGEMM_OK;
+        if (!yes) g_last_error = last;
+        return yes;
+    };
+    if ((me || ne) && (!me || accepts(h->edge_rows, me, n)) && (!ne || accepts(h->edge_cols, m - me, ne)))
         consider(m - me, n - ne, (me ? bf16x6::strip_time_us(me, n, k) : 0.0) +
                                      (ne ? bf16x6::strip_time_us(m - me, ne, k) : 0.0));
     return p;
