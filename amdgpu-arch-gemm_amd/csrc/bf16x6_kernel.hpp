@@ -5,19 +5,29 @@
 // The split.  x = x1 + x2 + x3, x1 = bf16(x), x2 = bf16(x - x1), x3 = x - x1 -
 // x2: both differences are exact in FP32 and the last one has at most 8
 // significant bits, so the three terms hold all 24 bits of x.  The products
-// a3 b1, a2 b2, a1 b3, a2 b1, a1 b2, a1 b1 go, smallest first, into one FP32
-// accumulator by v_mfma_f32_32x32x16_bf16; a2 b3, a3 b2 and a3 b3, at most
-// 2^-24 |a b| each and of random sign, are left out.
+// a3 b1, a2 b2, a1 b3, a2 b1, a1 b2 go, smallest first, into one FP32 accumulator,
+// a1 b1 into another (v_mfma_f32_32x32x16_bf16), and the two are added after the
+// K loop; a2 b3, a3 b2 and a3 b3, together at most 2^-24 |a b| and of random
+// sign, are left out.
 //
-// Accuracy.  Against 64 bits this is no further off than the FP32 MFMAs
-// (v_mfma_f32_32x32x2_f32, one rounding per product) at every depth measured:
-// relative error of U[-1,1) products at K = 64 / 256 / 1024 / 4096 / 16384
-// 1.08e-7 / 2.34e-7 / 4.84e-7 / 1.00e-6 / 2.09e-6 against 1.44e-7 / 2.87e-7 /
-// 5.72e-7 / 1.15e-6 / 2.29e-6, and 5.3e-7 against 8.4e-7 for positive values
-// at K = 4096: 16 products meet in one accumulation instead of two.  (All nine
-// products give the same figures; the largest first costs 25% at K = 64.)
-// Each accumulation rounds towards minus infinity, a bias that grows with the
-// number of them, so the host keeps K per accumulator chain below a limit.
+// Accuracy.  a1 b1 has 16 bits, so few of its sums round, and the small
+// products' sums round 2^-8 lower.  (In one accumulator, as these kernels had
+// it first, each of the six products is rounded at the full sum's size, some bits
+// below it are cut off downwards, and operands with zeros were up to 2.07 times
+// further from 64 bits than on the FP32 MFMAs, v_mfma_f32_32x32x2_f32, which
+// round once per two products.)  Relative error (2-norm) against 64 bits, this
+// kernel / the FP32 kernel, M = N = 4096:
+//   N(0,1), K = 256 / 1024 / 4096 / 24576   8.9e-8 / 1.9e-7 / 4.0e-7 / 1.0e-6
+//                                           2.9e-7 / 5.7e-7 / 1.1e-6 / 2.8e-6
+//   |N|, any sign, the same                 8.4e-8 / 1.6e-7 / 3.0e-7 / 8.4e-7
+//                                           2.2e-7 / 4.3e-7 / 8.4e-7 / 2.4e-6
+//   K = 4096, A rectified / 256 / 16 / 2 nonzeros to a column of B
+//                                           3.2e-7 / 1.1e-7 / 3.4e-8 / 2.6e-8
+//                                           8.1e-7 / 2.9e-7 / 7.4e-8 / 3.1e-8
+// What stays behind is the product left out: an output of a single nonzero product
+// is 2.6e-8 off (at most 1.8 * 2^-24 of it), a correctly rounded one 2.5e-8; so are
+// outputs of a few nonzeros that fall into different K waves or ranges (1.04
+// times the FP32 kernel's at four).
 //
 // Range.  BF16 has FP32's exponents, so no value loses range, but the low
 // terms of a value below 2^-110 would fall under BF16's smallest subnormal:
@@ -31,9 +41,11 @@
 //
 // Rate.  Six BF16 products replace an FP32 MFMA step that takes 16 times as
 // long per product: 2.5 PFLOP/s / 6 = 419 TFLOP/s against 157.  What bounds
-// these kernels is power: at 4096^3 the clock falls to 1.78 GHz with the
-// matrix cores 75% busy (2.36 GHz on inputs of zeros, 326 TFLOP/s).  4096^3:
-// 565 us (243 TFLOP/s) against 902 us for the FP32 kernel.
+// these kernels is power.  4096^3: 635-645 us back to back
+// (213 TFLOP/s; the FP32 kernel 902), the matrix cores 68% busy at 1.82 GHz of 2.4.
+//
+// Registers.  Two accumulators are what a 256 x 256 tile has no registers for (512
+// KB a CU); with one it took 580 us at 4096^3, 10 to 20% less than 256 x 128 tiles.
 //
 // Data path per K tile of KS steps of 16:
 //   HBM --buffer_load--> VGPR (FP32) --split--> LDS, three BF16 planes --> MFMA
@@ -409,12 +421,6 @@ __global__ void __launch_bounds__(G::NT) __attribute__((amdgpu_waves_per_eu(G::O
         constexpr int PL = F32 ? 2 : 3;   // 16-byte pieces of 8 values of k
         constexpr int PD = G::PD;
         float ra[PD][G::UA][8], rb[PD][G::UB][8];
-#pragma unroll
-        for (int i = 0; i < WT0; ++i)
-#pragma unroll
-            for (int j = 0; j < WT1; ++j)
-#pragma unroll
-                for (int q = 0; q < 16; ++q) acc[i][j][q] = 0.0f;
 
         auto k_of = [&](int s) __attribute__((always_inline)) { return (first + (uint32_t)(s - has)) * DK; };
         struct Pieces { u32x4 v[3]; };
@@ -486,6 +492,14 @@ __global__ void __launch_bounds__(G::NT) __attribute__((amdgpu_waves_per_eu(G::O
         }
         __syncthreads();
 
+        f32x16 low[WT0][WT1];   // sums of the products below a1 b1
+#pragma unroll
+        for (int i = 0; i < WT0; ++i)
+#pragma unroll
+            for (int j = 0; j < WT1; ++j)
+#pragma unroll
+                for (int q = 0; q < 16; ++q) acc[i][j][q] = low[i][j][q] = 0.0f;
+
         struct FragA { u32x4 v[PL]; };
         struct FragB { u32x4 v[WT1][PL]; };
         auto read_a = [&](int buf_off, int sub, int i, FragA& f) __attribute__((always_inline)) {
@@ -516,10 +530,11 @@ __global__ void __launch_bounds__(G::NT) __attribute__((amdgpu_waves_per_eu(G::O
 #pragma unroll
                 for (int e = 0; e < 6; ++e)
 #pragma unroll
-                    for (int j = 0; j < WT1; ++j)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                            __builtin_bit_cast(bf16x8, fb.v[j][PB[e]]), __builtin_bit_cast(bf16x8, fa.v[PA[e]]),
-                            acc[i][j], 0, 0, 0);
+                    for (int j = 0; j < WT1; ++j) {
+                        f32x16& sum = e < 5 ? low[i][j] : acc[i][j];
+                        sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, fb.v[j][PB[e]]),
+                                                                      __builtin_bit_cast(bf16x8, fa.v[PA[e]]), sum, 0, 0, 0);
+                    }
             }
         };
 
@@ -527,10 +542,17 @@ __global__ void __launch_bounds__(G::NT) __attribute__((amdgpu_waves_per_eu(G::O
         // the unrolled tiles of one trip: register sets and operand buffers are compile-time
         constexpr int U = 2;
         static_assert(PD <= 2, "one or two register sets");
+        // Staggered waves stage either before or after they multiply: their
+        // operands are read ahead of the staging, and one set is enough.
+        constexpr bool STAGGERED = G::PINGPONG && !F32;
+        static_assert(!STAGGERED || (SUBS == 1 && STEPS % 2 == 0 && NBUF >= 3), "operands of a tile in two sets of A, one of B");
         FragA fa[2];
-        FragB fb[2];
-        read_b(0, 0, fb[0]);
-        read_a(0, 0, 0, fa[0]);
+        FragB fb[STAGGERED ? 1 : 2];
+        auto read_first = [&](int buf_off, FragA& a, FragB& b) __attribute__((always_inline)) {
+            read_b(buf_off, 0, b);
+            read_a(buf_off, 0, 0, a);
+        };
+        if (!STAGGERED) read_first(0, fa[0], fb[0]);
         int cur = 0;                               // LDS offset of tile t's buffer
         int fill = (NBUF - 1) * G::STAGE;          // of the buffer tile t + NBUF - 1 goes to
         auto body = [&](int t, auto uu_tag, auto order_tag) __attribute__((always_inline)) {
@@ -548,6 +570,7 @@ __global__ void __launch_bounds__(G::NT) __attribute__((amdgpu_waves_per_eu(G::O
                 }
             };
             if constexpr (ORDER == 1) {
+                read_first(cur, fa[0], fb[0]);
                 stage_all();
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -558,7 +581,7 @@ __global__ void __launch_bounds__(G::NT) __attribute__((amdgpu_waves_per_eu(G::O
                 for (int i = 0; i < WT0; ++i) {
                     const int step = sub * WT0 + i;
                     const int as = (step + UU * STEPS) & 1;     // operand sets of this step
-                    const int bs = (sub + UU * SUBS) & 1;
+                    const int bs = STAGGERED ? 0 : (sub + UU * SUBS) & 1;
                     const bool last = step + 1 == STEPS;
                     int reads = 0, items = 0, vmem = 0;
                     if (!last) {
@@ -566,13 +589,12 @@ __global__ void __launch_bounds__(G::NT) __attribute__((amdgpu_waves_per_eu(G::O
                         if (i + 1 < WT0) {
                             read_a(cur, sub, i + 1, fa[as ^ 1]);
                         } else {
-                            read_b(cur, sub + 1, fb[bs ^ 1]);
+                            read_b(cur, sub + 1, fb[STAGGERED ? 0 : bs ^ 1]);
                             read_a(cur, sub + 1, 0, fa[as ^ 1]);
                             reads += PL * WT1;
                         }
-                    } else if (NBUF >= 3) {
-                        read_b(nxt, 0, fb[bs ^ 1]);
-                        read_a(nxt, 0, 0, fa[as ^ 1]);
+                    } else if (NBUF >= 3 && !STAGGERED) {
+                        read_first(nxt, fa[as ^ 1], fb[STAGGERED ? 0 : bs ^ 1]);
                         reads = PL + PL * WT1;
                     }
 #pragma unroll
@@ -605,18 +627,19 @@ __global__ void __launch_bounds__(G::NT) __attribute__((amdgpu_waves_per_eu(G::O
             if constexpr (ORDER != 0) __builtin_amdgcn_s_setprio(0);
             if constexpr (ORDER == 2) {
                 __builtin_amdgcn_sched_barrier(0);
+                read_first(nxt, fa[0], fb[0]);
                 stage_all();
             }
             fill = cur;
             cur = nxt;
             __syncthreads();
-            if (NBUF == 2) {
+            if constexpr (NBUF == 2) {
                 constexpr int as = (STEPS + UU * STEPS) & 1, bs = (SUBS + UU * SUBS) & 1;
-                read_b(cur, 0, fb[bs]);
-                read_a(cur, 0, 0, fa[as]);
+                read_first(cur, fa[as], fb[bs]);
             }
         };
         auto run = [&](auto order_tag) __attribute__((always_inline)) {
+            if constexpr (decltype(order_tag)::value == 2) read_first(cur, fa[0], fb[0]);
             for (int t = 0; t < tiles; t += U) {
                 body(t, Int<0>{}, order_tag);
                 if (t + 1 < tiles) body(t + 1, Int<1>{}, order_tag);
@@ -627,6 +650,14 @@ __global__ void __launch_bounds__(G::NT) __attribute__((amdgpu_waves_per_eu(G::O
             else run(Int<2>{});
         } else {
             run(Int<0>{});
+        }
+        if constexpr (!F32) {
+#pragma unroll
+            for (int i = 0; i < WT0; ++i)
+#pragma unroll
+                for (int j = 0; j < WT1; ++j)
+#pragma unroll
+                    for (int q = 0; q < 16; ++q) acc[i][j][q] += low[i][j][q];
         }
     };
 

@@ -1,11 +1,13 @@
 // When, and in which tile and K split, sgemm_launch runs the split-BF16
 // kernels of sgemm_bf16x6.hip instead of the handle's FP32 ones: a time model of
-// both, fitted to timings of 216 shapes on an MI355X (the package's workloads,
-// cubes from 512 to 6144, thin, tall, deep, shallow and ragged shapes in all
-// four layouts, C read or not; rms error 3-5% per tile, 12% for the FP32
-// kernels).  Over the 183 of them past kMinFlops the choice runs at 1.27 times
-// the FP32 kernels' speed (geometric mean), within 1.3% of always knowing the
-// fastest.  Host only; no HIP.
+// both, fitted to back-to-back launches of 216 shapes on an MI355X (the package's
+// workloads, cubes from 512 to 6144, thin, tall, deep, shallow and ragged shapes in
+// all four layouts, C read or not).  Over 220 other shapes drawn from the same
+// ranges its times are within 5-8% rms of the measured ones (K splits the most;
+// FP32 kernels 12%), and the 155 that it gives to the split kernels run at
+// 1.25 times the FP32 kernels' speed (geometric mean).  Launches with pauses
+// between them start on a faster clock and take up to a fifth less time than it
+// says.  Host only; no HIP.
 #pragma once
 
 #include <algorithm>
@@ -22,9 +24,8 @@ constexpr uint32_t kMinRange = 128;             // k values of one range, at lea
 // Leading dimensions below this keep one tile's span of every operand below
 // 2^31 bytes (256 rows or columns of 4 bytes).
 constexpr uint32_t kMaxLd = 1u << 21;
-// k values per accumulator chain, at most: the accumulation's bias overtakes
-// the FP32 kernels' random error (which grows with the square root) past
-// 32768: at 16384 2.09e-6 against 2.29e-6, at 65536 about 5.0e-6 against 4.6e-6
+// k values per accumulator chain, at most: as far as the errors of every sign
+// pattern are measured (0.36 of the FP32 kernels' at 24500)
 constexpr uint64_t kMaxChain = 24576;
 
 // One kernel: its tile, the K waves of a work-group (chains per range) and its
@@ -37,7 +38,6 @@ struct Tile {
     double launch, step_few, step_full, trans_a, fixed, store, read_c, partial;
 };
 constexpr Tile kTiles[] = {
-    {256, 256, 1, 4.42, 1.56, 2.16, 1.07, 4.28, 25.1, 32.9, 8.69},
     {128, 128, 2, 2.68, 0.484, 0.678, 1.0, 5.18, 4.0, 34.0, 9.01},
     {128, 64, 4, 2.07, 0.307, 0.399, 1.0, 4.34, 0.0, 31.6, 12.9},
     {256, 128, 1, 3.81, 0.898, 1.25, 1.015, 4.78, 9.9, 34.5, 8.79},
@@ -69,8 +69,7 @@ inline double time_us(const Tile& t, uint32_t splits, uint64_t m, uint64_t n, ui
     double us = t.launch + (double)full * round(1.0) + (part > 0.0 ? round(part) : 0.0);
     if (splits > 1) us += t.partial * (2 + splits) * mb;
     // near ties go to the launch without a workspace, which a handle's first
-    // split launch allocates, and to few ranges: with more the model is 2-3%
-    // too fast (128 x 64 tiles in 7 .. 10 ranges)
+    // split launch allocates, and to few ranges, where the model is closer
     if (splits > 1) us *= splits > 4 ? 1.04 : 1.02;
     const double bytes = 4.0 * ((double)m * k + (double)k * n + (double)m * n * (reads_c ? 2 : 1));
     return std::max(us, bytes / kBytesPerUs + t.launch);

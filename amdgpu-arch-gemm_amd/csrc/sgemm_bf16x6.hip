@@ -1,21 +1,17 @@
 // The library's split-BF16 kernels: the instances of bf16x6_kernel.hpp, in the
 // tile order of bf16x6_plan.hpp, for the four operand layouts.
 //
-//   256 x 256  eight waves of 128 x 64, K tiles of 16 in three LDS buffers
-//              (147 KB): 2.2 split operations per MFMA, the fewest, and the
-//              fastest wherever its tiles fill the GPU (4096^3: 243 TFLOP/s)
-//   256 x 128  eight waves of 64 x 64: grids that fill whole rounds only with
-//              smaller tiles (4096^3: 217 TFLOP/s)
+//   256 x 128  eight waves of 64 x 64, K tiles of 16 in three LDS buffers: the
+//              fewest split operations per MFMA, and the fastest wherever its
+//              tiles fill the GPU (4096^3: 213 TFLOP/s)
 //   128 x 128  two groups of four 64 x 64 waves, each multiplying every other
-//              step of 16 (2048^3: 91 us, against 132 in 256 x 128 tiles and
-//              112 in the four-wave kernel with two work-groups per CU)
+//              step of 16 (2048^3: 91 us, against 132 in 256 x 128 tiles)
 //   128 x 64   four groups of two 64 x 64 waves: few output tiles
-//              (512 x 512 x 16384: 62 us with 8 K ranges)
+//              (511 x 513 x 16400 in 6 K ranges)
 //
-// The two-group kernels stagger their waves: half of them splits the next
-// tile's operands while the other half multiplies (2048^3: 89 us against 93,
-// 4096^3 in 128 x 128 tiles 676 against 712; 256 x 256 has no registers for it
-// and gains nothing, being limited by power).
+// The first two stagger their waves: half of them splits the next tile's
+// operands while the other half multiplies (2048^3: 91 us against 92, 8192^3 TT
+// 5226 against 5441).
 
 #include "bf16x6_kernel.hpp"
 #include "bf16x6_plan.hpp"
@@ -33,7 +29,6 @@ using bf16x6::Config;
 
 //                                          waves      tiles  K
 //                                          m  n  k    m  n   steps, buffers, register sets; group; waves per SIMD; staggered
-template <bool TA, bool TB> using T256x256 = Config<2, 4, 1, 4, 2, 1, 3, 1, 4, 2, 0, TA, TB>;
 template <bool TA, bool TB> using T128x128 = Config<2, 2, 2, 2, 2, 2, 3, 1, 4, 2, 1, TA, TB>;
 template <bool TA, bool TB> using T128x64 = Config<2, 1, 4, 2, 2, 4, 2, 1, 8, 2, 0, TA, TB>;
 template <bool TA, bool TB> using T256x128 = Config<4, 2, 1, 2, 2, 1, 3, 1, 4, 2, 1, TA, TB>;
@@ -43,7 +38,7 @@ template <template <bool, bool> class T, int INDEX> constexpr bool matches() {
     return G::MT0 == bf16x6::kTiles[INDEX].m && G::MT1 == bf16x6::kTiles[INDEX].n &&
            G::KW == bf16x6::kTiles[INDEX].k_waves;
 }
-static_assert(matches<T256x256, 0>() && matches<T128x128, 1>() && matches<T128x64, 2>() && matches<T256x128, 3>(),
+static_assert(matches<T128x128, 0>() && matches<T128x64, 1>() && matches<T256x128, 2>(),
               "the instances follow the plan's tile order");
 
 constexpr int kMaxDevices = 64;
@@ -77,10 +72,9 @@ int sgemm_internal::bf16x6_launch(int tile, uint32_t splits, bool trans_a, bool 
     p.tickets = tickets;
     p.splits = splits;
     hipError_t e = hipErrorInvalidValue;
-    if (tile == 0) e = launch_tile<T256x256>(trans_a, trans_b, p, stream);
-    else if (tile == 1) e = launch_tile<T128x128>(trans_a, trans_b, p, stream);
-    else if (tile == 2) e = launch_tile<T128x64>(trans_a, trans_b, p, stream);
-    else if (tile == 3) e = launch_tile<T256x128>(trans_a, trans_b, p, stream);
+    if (tile == 0) e = launch_tile<T128x128>(trans_a, trans_b, p, stream);
+    else if (tile == 1) e = launch_tile<T128x64>(trans_a, trans_b, p, stream);
+    else if (tile == 2) e = launch_tile<T256x128>(trans_a, trans_b, p, stream);
     if (e == hipSuccess) return SGEMM_OK;
     char msg[160];
     snprintf(msg, sizeof(msg), "launch of the split-BF16 kernel failed: %s (%d)", hipGetErrorString(e), (int)e);
@@ -94,7 +88,7 @@ int sgemm_internal::bf16x6_prepare() {
     std::lock_guard<std::mutex> lock(g_mutex);
     if (dev >= 0 && g_loaded[dev]) return SGEMM_OK;
     hipFuncAttributes a;
-    const hipError_t e = hipFuncGetAttributes(&a, reinterpret_cast<const void*>(&bf16x6::kernel<T256x256<false, false>>));
+    const hipError_t e = hipFuncGetAttributes(&a, reinterpret_cast<const void*>(&bf16x6::kernel<T256x128<false, false>>));
     if (e == hipSuccess) {
         if (dev >= 0) g_loaded[dev] = true;
         return SGEMM_OK;
