@@ -564,8 +564,8 @@ int decompose(const sgemm_handle* h, uint32_t m, uint32_t n, uint32_t k, uint32_
 }
 
 thin::Shape thin_shape(const sgemm_handle* h, uint32_t m, uint32_t n, uint32_t k, uint32_t lda, uint32_t ldb) {
-    if (!h->split_bf16 || h->fixed_split || h->fixed_stream || !thin_launch) return thin::Shape();
-    return thin::choose(m, n, k, lda, ldb, h->info.trans_a != 0, h->info.trans_b != 0);
+    if (!h->split_bf16 || h->fixed_split || h->fixed_stream || !thin_launch || h->compute_units <= 0) return thin::Shape();
+    return thin::choose(m, n, k, lda, ldb, h->info.trans_a != 0, h->info.trans_b != 0, h->compute_units);
 }
 
 SplitPlan split_plan(const sgemm_handle* h, uint32_t m, uint32_t n, uint32_t k, uint32_t lda, uint32_t ldb, uint32_t ldc,

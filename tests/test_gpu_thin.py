@@ -119,3 +119,45 @@ def test_every_thin_shape_has_a_kernel(tmp_path):
     csrc = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "amdgpu-arch-gemm_amd", "csrc")
     subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-I", csrc, str(src), "-o", str(exe)], check=True)
     assert subprocess.run([str(exe)]).returncode == 0
+
+
+ROUNDS = r"""
+#include "thin_plan.hpp"
+#include <cstdio>
+#include <random>
+static bool on(uint32_t m, uint32_t n, uint32_t k, bool ta, bool tb, int cus) {
+    return thin::choose(m, n, k, ta ? k : m, tb ? n : k, ta, tb, cus).on;
+}
+int main() {
+    // one grid, one time: every row count of a whole round's last work-groups takes the same route
+    for (uint32_t rows = 16353; rows <= 16384; ++rows)
+        if (!on(rows, 16, 8192, true, false, 256)) { std::printf("%u rows\n", rows); return 1; }
+    // a second round of a few work-groups takes as long as a full one, and on another chip begins elsewhere
+    if (!on(4096, 16, 4096, true, false, 256) || on(4400, 16, 4096, true, false, 256) || !on(4400, 16, 4096, true, false, 304)) return 2;
+    // within one grid more rows cost the thin kernel nothing: a route taken is kept
+    std::mt19937 rng(11);
+    int taken = 0;
+    for (int i = 0; i < 200000; ++i) {
+        const uint32_t step = 64, base = 1024 + step * (rng() % 300), cols = 1 + rng() % 16, k = 256 + rng() % 9000;
+        const bool ta = i & 1, tb = i & 2;
+        const uint32_t lo = base + 1 + rng() % (step - 1), hi = base + step;
+        if (base == 4736 || base == 6080 || base == 8128) continue;   // the tile's width changes
+        if ((lo * 4e-6 * k > 256.0) != (hi * 4e-6 * k > 256.0)) continue;   // the last-level cache ends
+        const thin::Shape a = thin::choose(lo, cols, k, ta ? k : lo, tb ? cols : k, ta, tb), b = thin::choose(hi, cols, k, ta ? k : hi, tb ? cols : k, ta, tb);
+        const uint32_t w = 16u * (uint32_t)(a.x_atoms > 0 ? a.x_atoms : 1);
+        if ((lo + w - 1) / w != (hi + w - 1) / w) continue;
+        taken += a.on;
+        if (a.on && !b.on) { std::printf("%u on, %u off: %u x %u\n", lo, hi, cols, k); return 3; }
+    }
+    return taken > 10000 ? 0 : 4;
+}
+"""
+
+
+def test_the_route_follows_the_rounds_of_work_groups(tmp_path):
+    src, exe = tmp_path / "rounds.cpp", tmp_path / "rounds"
+    src.write_text(ROUNDS)
+    csrc = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "amdgpu-arch-gemm_amd", "csrc")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-I", csrc, str(src), "-o", str(exe)], check=True)
+    ret = subprocess.run([str(exe)], stdout=subprocess.PIPE)
+    assert ret.returncode == 0, (ret.returncode, ret.stdout.decode())
