@@ -12,13 +12,15 @@ NAME = "mt64x64_a16_wg1x4_dk32_s3"
 
 
 def test_noalloc_on_streams_that_take_turns(kernels):
-    # partials of 0.6, 4 and 0.1 MB in slots of 4 MB, and one that takes all 32 MB's slots
-    shapes = [(333, 129, 517), (256, 256, 4096), (70, 45, 1001), (448, 448, 16384)]
+    # partials of 0.6, 4 and 0.1 MB in slots of 4 MB, and 8 MB, which take all of them
+    shapes = [(333, 129, 517), (256, 256, 4096), (70, 45, 1001), (640, 640, 8192)]
     bufs, want = [], []
     with S.Kernel(*catalog.paths(NAME)) as ref:
         for i, (m, n, k) in enumerate(shapes):
             ref.set_split_bf16(0)
             assert ref.launch_splits(m, n, k) > 1
+            # a slot is an eighth of the scratch; the workspace's size counts its tickets too
+            assert (ref.workspace_size(m, n, k) > S.SGEMM_NOALLOC_PARTIAL_BYTES // 8 + 4096) == (i == 3)
             bufs.append([S.DeviceBuffer.from_array(S.fill_matrix(*s, 60 + i, j))
                          for j, s in enumerate(((m, k), (k, n)))] + [S.DeviceBuffer(4 * m * n)])
             ref.launch(bufs[i][0], bufs[i][1], None, bufs[i][2], m, n, k)

@@ -468,19 +468,24 @@ def test_baseline_config(kernels, cid, m, n, k, seed, dist):
     _say(f"config {cid} {m}x{n}x{k} seed {seed} dist {dist} -> {name}")
     A = S.fill_matrix(m, k, seed, 0, dist)
     B = S.fill_matrix(k, n, seed, 1, dist)
+    outs = {}
     with _kernel(name) as kern:
-        D, ms = kern.run(A, B, None, m, n, k, alpha=1.0, beta=0.0, warmup=1, runs=3)
-    _say(f"  {ms:.3f} ms/run, {2.0 * m * n * k / ms * 1e-9:.1f} TFLOP/s")
-    assert np.all(np.isfinite(D))
+        for what, mode in (("as selected", 1), ("FP32 kernel", 0)):   # the split-BF16 kernels run the first where they are faster
+            kern.set_split_bf16(mode)
+            plan = kern.split_bf16_plan(m, n, k)
+            outs[what], ms = kern.run(A, B, None, m, n, k, alpha=1.0, beta=0.0, warmup=1, runs=3)
+            _say(f"  {what}: split-BF16 plan {plan}, {ms:.3f} ms/run, {2.0 * m * n * k / ms * 1e-9:.1f} TFLOP/s")
+            assert np.all(np.isfinite(outs[what])) and (mode or plan is None)
     ref = oracle.cpu_gemm_blocked(A, B, None, 1.0, 0.0, threads=16)
-    err = _check(D, ref, k, f"{cid} whole D vs cpuGemm")
     ref64 = np.asarray(A, dtype=np.float64) @ np.asarray(B, dtype=np.float64)
-    err64 = _check(D, ref64, k, f"{cid} whole D vs float64")
     cpu64 = oracle.normwise_error(ref, ref64)
-    mismatches = int(np.count_nonzero(~(np.abs(D - ref) < np.float32(1e-3))))
-    _say(f"  whole D ({m * n} outputs): normwise error {err:.3e} vs cpuGemm, {err64:.3e} vs float64 "
-         f"(cpuGemm itself {cpu64:.3e}), tolerance {oracle.tolerance(k):.3e}; "
-         f"|gpu - cpu| >= 1e-3 at {mismatches} of {m * n}, max |gpu - cpu| {float(np.max(np.abs(D - ref))):.3e}")
+    for what, D in outs.items():
+        err = _check(D, ref, k, f"{cid} whole D vs cpuGemm, {what}")
+        err64 = _check(D, ref64, k, f"{cid} whole D vs float64, {what}")
+        mismatches = int(np.count_nonzero(~(np.abs(D - ref) < np.float32(1e-3))))
+        _say(f"  {what}: whole D ({m * n} outputs): normwise error {err:.3e} vs cpuGemm, {err64:.3e} vs float64 "
+             f"(cpuGemm itself {cpu64:.3e}), tolerance {oracle.tolerance(k):.3e}; "
+             f"|gpu - cpu| >= 1e-3 at {mismatches} of {m * n}, max |gpu - cpu| {float(np.max(np.abs(D - ref))):.3e}")
 
 
 # ----------------------------------------------------- wave specialisation
