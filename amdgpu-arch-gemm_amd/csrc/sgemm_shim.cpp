@@ -1023,10 +1023,11 @@ int sgemm_launch(sgemm_handle* h, const float* dA, const float* dB, const float*
                                            ldb, ldc, ldd, alpha, beta, h->stream);
     sgemm_internal::Part parts[3];
     sgemm_internal::SplitPlan sp = sgemm_internal::split_plan(h, m, n, k, lda, ldb, ldc, ldd, alpha, beta);
-    // A plan whose workspace cannot be had (under capture, which no allocation
-    // may join, or for want of memory) leaves the call to h's own kernels, which
-    // may need none.
-    if (sp.tile >= 0 && (h->ws_bytes < sp.partial_bytes || h->ticket_count < sp.ticket_count) &&
+    // A plan that needs a workspace leaves the call to h's own kernels, which may
+    // need none, for want of memory and under capture: no allocation may join a
+    // graph, and its replays must not hold on to a workspace that a later,
+    // larger launch replaces, or share it with launches on other streams.
+    if (sp.partial_bytes &&
         (is_capturing(h->stream) || grow_workspace(h, h->stream, sp.partial_bytes, sp.ticket_count) != SGEMM_OK))
         sp = sgemm_internal::SplitPlan();
     int count = sp.tile >= 0 ? sgemm_internal::split_strips(h, sp, m, n, lda, ldb, ldc, ldd, parts)

@@ -253,9 +253,9 @@ int sgemm_memset(void* dptr, int value, size_t bytes);
  * instead (or, under sgemm_set_stream_k, the stream-K kernel), with the handle's
  * workspace; launches of one handle share that
  * workspace, so they must run in order on the handle's stream.  A launch whose
- * workspace is larger than the handle's allocates it; under graph capture, where
- * that is not possible, a split-BF16 launch (sgemm_set_split_bf16) leaves the
- * call to h's own kernels, which may need none.  Device
+ * workspace is larger than the handle's allocates it; under graph capture a
+ * split-BF16 launch (sgemm_set_split_bf16) that needs one leaves the call to h's
+ * own kernels, which may need none (sgemm_launch_noalloc captures it).  Device
  * pointers need 4-byte alignment only (SGEMM_E_INVALID otherwise). */
 int sgemm_launch(sgemm_handle* h, const float* dA, const float* dB, const float* dC, float* dD,
                  uint32_t m, uint32_t n, uint32_t k, uint32_t lda, uint32_t ldb, uint32_t ldc, uint32_t ldd,

@@ -20,7 +20,7 @@ def _bits(m, n, k, entry, kern, a, b, d):
 
 @pytest.mark.parametrize("entry,m,n,k,warm", [
     ("launch", 16384, 128, 4096, False),         # needs no workspace on the FP32 kernel, K ranges on the split one
-    ("launch", 16384, 128, 4096, True),          # the handle holds the workspace already
+    ("launch", 16384, 128, 4096, True),          # the handle holds the workspace already, until a larger launch replaces it
     ("launch_noalloc", 16384, 128, 4096, False),
     ("launch_noalloc", 1000, 999, 4097, False),
     ("launch", 2048, 2048, 1024, False),         # no K split
@@ -47,8 +47,12 @@ def test_captured_split_launches_replay(kernels, entry, m, n, k, warm):
             getattr(kern, entry)(a, b, None, d, m, n, k)
         finally:
             exe = hip.end(stream)
-        # a cold handle has no workspace for the K ranges and cannot allocate it under capture
-        want = own if entry == "launch" and plan["splits"] > 1 and not warm else split
+        # a graph of sgemm_launch uses no workspace: the handle cannot allocate it under capture, and may replace it later
+        want = own if entry == "launch" and plan["splits"] > 1 else split
+        if warm:
+            assert kern.workspace_size(1536, 1536, 1531) > kern.workspace_size(m, n, k)
+            large = [S.DeviceBuffer(4 * 1536 * 1536) for _ in range(3)]
+            kern.launch(*large[:2], None, large[2], 1536, 1536, 1531)
         for q in range(3):
             d.upload(np.full(m * n, np.nan, dtype=np.float32))
             _ok(hip.lib.hipGraphLaunch(exe, stream))
