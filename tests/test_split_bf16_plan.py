@@ -57,14 +57,15 @@ def test_every_choice_fits_the_scratch_and_the_chain_rules(tmp_path):
     assert ret.returncode == 0, ret.stdout.decode()
 
 
-STRIPS = r"""
+HOST = r"""
 #include "sgemm_shim.cpp"
 #include <cmath>
 #include <random>
+static int split_launches = 0;
 int sgemm_internal::noalloc_prepare(int) { return SGEMM_OK; }
 int sgemm_internal::bf16x6_launch(int, uint32_t, bool, bool, const float*, const float*, const float*, float*, uint32_t,
                                   uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, float, float, float*,
-                                  uint32_t*, hipStream_t) { return SGEMM_OK; }
+                                  uint32_t*, hipStream_t) { ++split_launches; return SGEMM_OK; }
 int sgemm_internal::bf16x6_prepare() { return SGEMM_OK; }
 int sgemm_internal::thin_prepare() { return SGEMM_OK; }
 int sgemm_internal::thin_launch(const thin::Shape&, bool, bool, const float*, const float*, const float*, float*, uint32_t,
@@ -77,6 +78,9 @@ static sgemm_handle* handle(int tm, int tn, int dk) {
     h->compute_units = 256; h->resident = 256; h->split_bf16 = true;
     return h;
 }
+"""
+
+STRIPS = HOST + r"""
 int main() {
     // the catalog's 256 x 256 instance and its edge pair
     sgemm_handle *h = handle(256, 256, 24), *rows = handle(16, 128, 64), *cols = handle(64, 16, 64);
@@ -105,12 +109,9 @@ int main() {
 """
 
 
-def test_no_strip_goes_to_an_edge_kernel_that_refuses_it(tmp_path):
-    """A launch that the handle's own kernel accepts is not refused for a strip
-    that the split plan alone would cut (the edge kernel's grid ends at 65535
-    of its narrower tiles)."""
-    src, exe = tmp_path / "strips.cpp", tmp_path / "strips"
-    src.write_text(STRIPS)
+def _build_and_run(tmp_path, name, text):
+    src, exe = tmp_path / (name + ".cpp"), tmp_path / name
+    src.write_text(text)
     csrc = os.path.join(ROOT, "amdgpu-arch-gemm_amd", "csrc")
     rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
     subprocess.run(["g++", "-std=c++17", "-O1", "-D__HIP_PLATFORM_AMD__", "-I", csrc, "-I", os.path.join(ROOT, "include"), "-I",
@@ -118,3 +119,60 @@ def test_no_strip_goes_to_an_edge_kernel_that_refuses_it(tmp_path):
                     "-Wl,-rpath," + os.path.join(rocm, "lib"), "-pthread"], check=True)
     ret = subprocess.run([str(exe)], stdout=subprocess.PIPE)
     assert ret.returncode == 0, (ret.returncode, ret.stdout.decode())
+
+
+def test_no_strip_goes_to_an_edge_kernel_that_refuses_it(tmp_path):
+    """A launch that the handle's own kernel accepts is not refused for a strip
+    that the split plan alone would cut (the edge kernel's grid ends at 65535
+    of its narrower tiles)."""
+    _build_and_run(tmp_path, "strips", STRIPS)
+
+
+# HIP calls that sgemm_launch makes, answered here
+WORKSPACE = HOST + r"""
+static bool capturing = false, memory = true;
+static int own_launches = 0, allocations = 0;
+static char block[64];
+extern "C" {
+hipError_t hipMalloc(void** p, size_t) { if (!memory) return hipErrorOutOfMemory; ++allocations; *p = block; return hipSuccess; }
+hipError_t hipFree(void*) { return hipSuccess; }
+hipError_t hipMemsetAsync(void*, int, size_t, hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return capturing ? hipErrorStreamCaptureUnsupported : hipSuccess; }
+hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* s) {
+    *s = capturing ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
+    return hipSuccess;
+}
+hipError_t hipModuleLaunchKernel(hipFunction_t, unsigned, unsigned, unsigned, unsigned, unsigned, unsigned, unsigned,
+                                 hipStream_t, void**, void**) { ++own_launches; return hipSuccess; }
+}
+int main() {
+    // 16384 x 128 x 4096: 256 tiles of 128 x 64, no K ranges on the handle's own kernel
+    sgemm_handle* h = handle(128, 64, 64);
+    const uint32_t m = 16384, n = 128, k = 4096;
+    float *a = (float*)(1ull << 40), *b = a + (1u << 28), *d = b + (1u << 28);
+    const sgemm_internal::SplitPlan p = sgemm_internal::split_plan(h, m, n, k, m, k, m, m, 1.0f, 0.0f);
+    if (p.tile < 0 || p.splits < 2 || sgemm_internal::plan(h, m, n, k).partial_bytes) return 2;
+    auto launch = [&](int split, int own) {
+        split_launches = own_launches = 0;
+        const int r = sgemm_launch(h, a, b, nullptr, d, m, n, k, m, k, m, m, 1.0f, 0.0f);
+        if (r == SGEMM_OK && split_launches == split && own_launches == own) return true;
+        std::printf("returned %d (%s), %d split, %d own launches, expected %d, %d\n", r, sgemm_last_error(), split_launches,
+                    own_launches, split, own);
+        return false;
+    };
+    capturing = true;
+    if (!launch(0, 1) || allocations) return 3;    // the first launch, captured
+    capturing = false, memory = false;
+    if (!launch(0, 1)) return 4;                   // no memory for the workspace
+    memory = true;
+    if (!launch(1, 0) || allocations != 2) return 5;
+    if (!launch(1, 0) || allocations != 2) return 6;
+    capturing = true;
+    if (!launch(0, 1)) return 7;                   // a graph holds no workspace
+    return 0;
+}
+"""
+
+
+def test_a_split_launch_without_a_workspace_runs_the_handles_own_kernel(tmp_path):
+    _build_and_run(tmp_path, "workspace", WORKSPACE)
