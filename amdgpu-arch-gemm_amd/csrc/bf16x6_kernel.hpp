@@ -41,8 +41,9 @@
 //
 // Rate.  Six BF16 products replace an FP32 MFMA step that takes 16 times as
 // long per product: 2.5 PFLOP/s / 6 = 419 TFLOP/s against 157.  What bounds
-// these kernels is power.  4096^3: 635-645 us back to back
-// (213 TFLOP/s; the FP32 kernel 902), the matrix cores 68% busy at 1.82 GHz of 2.4.
+// these kernels is power, and between the matrix instructions the splitting and the
+// LDS: 4096^3 635-645 us back to back (213 TFLOP/s; the FP32 kernel 902), the matrix
+// cores 68% busy at 1.82 GHz of 2.4.
 //
 // Registers.  Two accumulators are what a 256 x 256 tile has no registers for (512
 // KB a CU); with one it took 580 us at 4096^3, 10 to 20% less than 256 x 128 tiles.
@@ -323,14 +324,15 @@ __device__ __forceinline__ void finish(const Args& p, unsigned char* lds, f32x16
     // Element e of chunk (j * 4 + h) * WT0 + i: row i * 32 + r, column j * 32 + 8 h + 4 g + e,
     // one dword per lane: 32 consecutive rows, whole 128-byte lines.  Columns
     // past n lie past the descriptor's end, rows past m get an offset that
-    // does: the range check drops both, so edge tiles run the same code.
+    // does: the range check, which counts the scalar offset too, drops both, so edge
+    // tiles run the same code.
     constexpr uint32_t NOWHERE = 0x80000000u;
     const uint32_t voc = ((uint32_t)(4 * g) * p.ldc + (uint32_t)r) * 4u, vod = ((uint32_t)(4 * g) * p.ldd + (uint32_t)r) * 4u;
     static_assert(G::OWN % WT0 == 0, "a share holds every atom along m");
     // With one wave's stores down whole columns the L2 joins the pieces of a
-    // line that columns off a 128-byte boundary leave (5399 x 4428 x 267 in 256 x
-    // 256 tiles: 92 us, against 105 with streaming stores and 130 with the atoms'
-    // rows stored far apart); shares of K waves are spread thinner and gain
+    // line that columns off a 128-byte boundary leave (5399 x 4428 x 267 in
+    // tiles of 256 x 256, which are gone: 92 us, against 105 with streaming stores and
+    // 130 with the atoms' rows stored far apart); shares of K waves are spread thinner and gain
     // 2-3% from streaming.
     constexpr int STORE_POLICY = KW > 1 ? CPOL_NT : 0;
     auto chunk_row = [&](int c) __attribute__((always_inline)) { return (uint32_t)(c % WT0) * 32u; };
