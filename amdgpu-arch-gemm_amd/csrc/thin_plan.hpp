@@ -18,6 +18,7 @@ struct Shape {
 constexpr uint32_t kMaxCols = 16;
 constexpr uint32_t kMaxLd = 1u << 21;     // 64 rows or 64 k of it are a 32-bit byte offset
 constexpr uint32_t kMinRows = 1024;       // 64 work-groups
+constexpr uint32_t kMaxRows = 1u << 27;   // 2^23 work-groups of 256: a grid holds fewer than 2^32 work-items
 constexpr uint32_t kMinDepth = 256;       // a chunk for each of four waves
 constexpr uint32_t kMaxDepth = 16384;     // a wave's FP32 chain is at most 2048 long, as far as errors are measured
 
@@ -45,7 +46,7 @@ inline Shape choose(uint32_t m, uint32_t n, uint32_t k, uint32_t lda, uint32_t l
     if (std::max(lda, ldb) >= kMaxLd || k < kMinDepth || k > kMaxDepth) return t;
     t.x_is_a = n <= m;
     const uint32_t rows = t.x_is_a ? m : n, cols = t.x_is_a ? n : m;
-    if (cols > kMaxCols || rows < kMinRows) return t;
+    if (cols > kMaxCols || rows < kMinRows || rows > kMaxRows) return t;
     const bool xkc = t.x_is_a ? trans_a : !trans_b, ykc = t.x_is_a ? !trans_b : trans_a;
     // Wider tiles read Y less often, narrower ones make more work-groups.  X
     // contiguous in k: two atoms gain with many rows and a Y that is read in

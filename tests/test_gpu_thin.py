@@ -134,6 +134,17 @@ int main() {
         if (!on(rows, 16, 8192, true, false, 256)) { std::printf("%u rows\n", rows); return 1; }
     // a second round of a few work-groups takes as long as a full one, and on another chip begins elsewhere
     if (!on(4096, 16, 4096, true, false, 256) || on(4400, 16, 4096, true, false, 256) || !on(4400, 16, 4096, true, false, 304)) return 2;
+    // a grid of 2^32 work-items cannot be launched (2^28 rows by 256 of k, A^T: 275 GB): the tile kernels take the call
+    for (uint64_t rows = 1u << 20; rows < 1u << 29; rows += 1u << 20)
+        for (uint32_t k : {256u, 512u, 1023u, 1024u, 4096u})
+            for (int layout = 0; layout < 2; ++layout) {
+                if (rows * k * 4 > 288000000000ull) continue;   // more than the device holds
+                const thin::Shape t = thin::choose((uint32_t)rows, 16, k, k, layout ? 16 : k, true, layout);
+                if (t.on && (rows + 16 * t.x_atoms - 1) / (16 * t.x_atoms) * 64u * t.waves >= 1ull << 32) {
+                    std::printf("%llu rows, k = %u: %d atoms, %d waves\n", (unsigned long long)rows, k, t.x_atoms, t.waves);
+                    return 5;
+                }
+            }
     // within one grid more rows cost the thin kernel nothing: a route taken is kept
     std::mt19937 rng(11);
     int taken = 0;
